@@ -277,12 +277,19 @@ constexpr int kCoreThreads = 64 * kCoreWaves;
 constexpr int kRows = 2;
 
 // Blocks are dispatched round-robin over the 8 XCDs.  A "column" is one
-// (head, query tile); every XCD owns a contiguous run of columns, so the
-// triangle-bias rows those columns re-read for every row group stay in that
-// XCD's L2 instead of being fetched again from HBM / MALL.
+// (head, query tile); every XCD owns a contiguous run of cols / 8 columns, so
+// the triangle-bias rows those columns re-read for every row group stay in
+// that XCD's L2 instead of being fetched again from HBM / MALL.  The items
+// (column, row group) of the cols % 8 columns left over are dealt out in eight
+// contiguous runs, so every XCD has the same number of blocks to within one
+// (whole columns only left 2 of 8 XCDs idle at 12 columns, n = 312, and one
+// XCD with a fifth of the work at 36, n = 1134).
 __host__ __device__ inline int core_qtiles(int n) { return (n + kCoreQ - 1) / kCoreQ; }
-__host__ __device__ inline int core_cols_per_xcd(int n) { return (kH * core_qtiles(n) + 7) / 8; }
 __host__ __device__ inline int core_row_groups(int n) { return (n + kRows - 1) / kRows; }
+__host__ __device__ inline int core_full_cols(int n) { return kH * core_qtiles(n) / 8; }  // per XCD
+__host__ __device__ inline int core_rest_items(int n) {  // per XCD, of the columns left over
+  return (kH * core_qtiles(n) % 8 * core_row_groups(n) + 7) / 8;
+}
 
 // LDS stage buffer, per block: K and V^T tiles of the kRows rows, every wave's
 // triangle-bias B tiles for the stage (4 tiles x 512 B), and the rows' mask
@@ -596,11 +603,18 @@ __global__ __launch_bounds__(kCoreThreads) __attribute__((amdgpu_waves_per_eu(4)
   __shared__ __attribute__((aligned(16))) char stage_lds[2 * kStageBytes];
   const int n = L.n, np = L.np;
   const int qtiles = core_qtiles(n);
-  const int cpx = core_cols_per_xcd(n);
-  const int bid = blockIdx.x;
-  const int idx = bid >> 3;
-  const int col = (bid & 7) * cpx + idx % cpx, ig = idx / cpx;
-  if (col >= kH * qtiles) return;  // uniform over the block
+  const int rgroups = core_row_groups(n), full = core_full_cols(n);
+  const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+  int col, ig;
+  if (idx < full * rgroups) {
+    col = xcd * full + idx % full;
+    ig = idx / full;
+  } else {
+    const int item = xcd * core_rest_items(n) + idx - full * rgroups;
+    col = 8 * full + item / rgroups;
+    ig = item % rgroups;
+    if (col >= kH * qtiles) return;  // the last run is shorter (uniform over the block)
+  }
   const int h = col / qtiles, qt = col % qtiles;
   const int t = threadIdx.x, w = t >> 6;
   const int i0 = ig * kRows;
@@ -817,7 +831,8 @@ int run(const TIn* x, const float* mask, int n, int starting, float inf, const f
     if (int rc = check_launch("triattn_proj")) return rc;
   }
   if (stages & 2) {
-    triattn_core_kernel<<<dim3((unsigned)(8ll * core_cols_per_xcd(n) * core_row_groups(n))), kCoreThreads, 0, st>>>(L);
+    const int64_t per_xcd = (int64_t)core_full_cols(n) * core_row_groups(n) + core_rest_items(n);
+    triattn_core_kernel<<<dim3((unsigned)(8 * per_xcd)), kCoreThreads, 0, st>>>(L);
     if (int rc = check_launch("triattn_core")) return rc;
   }
   if (stages & 4) {
