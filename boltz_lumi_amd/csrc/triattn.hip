@@ -19,8 +19,8 @@
 //  K3 triattn_out    o * sigmoid(linear_g(LN(x')) + b_g) -> linear_o + b_o, then
 //                    write or add into the fp32 residual in place.
 //
-// Workspace (np = round_up(n, 128)):
-//   q[i][h][j][d], k[i][h][j][d], vt[i][h][d][j']  bf16, i < np, j < np, where
+// Workspace (np = round_up(n, 256); nx = round_up(n, 64) rows and columns of it are used):
+//   q[i][h][j][d], k[i][h][j][d], vt[i][h][d][j']  bf16, i < nx, j < nx, where
 //     j' = (j & ~31) + vperm(j & 31) permutes keys inside each 32-key block
 //   tb: H x np x np bf16 in B-operand order (tb_offset; k >= n is kPadBias), mb[i][k] fp32,
 //   o[i][j][h*32+d] bf16 (n x n)
@@ -30,7 +30,13 @@ using namespace bmx;
 
 namespace {
 
-constexpr int kH = 4, kD = 32, kPad = 256;  // row padding: a multiple of the projection and attention tiles
+constexpr int kH = 4, kD = 32;
+// Row strides of the workspace are multiples of kPad; rows and columns are
+// written and read up to nx = round_up(n, 64) only (the projection's tile and
+// the core's key stage).  Projecting the whole np x np frame cost the padded
+// area: 48 us against 29 at n = 312, 140 against 93 at n = 576, 417 against 350
+// at n = 1134 (starting node).
+constexpr int kPad = 256;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kProjRows = 3 * kC + 32;  // q, k, v, then H triangle-bias rows (+ zero rows)
 // Triangle-bias storage type: bf16, as upstream's bf16 path rounds the bias.
@@ -43,7 +49,7 @@ using tb_t = bf16;
 constexpr float kPadBias = -1e30f;
 
 struct Layout {
-  int n, np;
+  int n, np, nx;
   bf16 *q, *k, *vt, *o;
   tb_t* tb;
   float* mb;
@@ -88,7 +94,7 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
 // Persistent and weight-stationary.  Wave w keeps head w's q, k and v weight
 // rows (3 x 32 rows, 32x32x16 operands) and the 4 triangle-bias rows (16x16x32
 // A operands) in VGPRs for the block's lifetime.  A tile is 64 positions
-// (i, j0..j0+63) of the row frame over the padded np x np range, so padding
+// (i, j0..j0+63) of the row frame over the padded nx x nx range, so padding
 // rows and keys get their zero / -inf values from the same code; the next
 // tile's input rows are prefetched into registers during the current tile's
 // MFMAs.  q, k and v^T leave through an LDS stage in their HBM order and are
@@ -114,7 +120,7 @@ __global__ __launch_bounds__(256, 2) void triattn_proj_kernel(const TIn* __restr
   const int t = threadIdx.x, l = lane_id(), w = t >> 6, h = w, g = l >> 4, lq = l & 15;
   const int hw = t >> 5, hl = t & 31;
   const LnAffine aff = ln_affine(ln_w, ln_b, hl);
-  const int tiles_x = np / kP1, total = np * tiles_x;
+  const int tiles_x = L.nx / kP1, total = L.nx * tiles_x;
   const float qscale = kLog2e / sqrtf((float)kD);
 
   // Weight rows: q, k, v of head h are rows 32h, 128 + 32h, 256 + 32h; the
@@ -342,6 +348,9 @@ __device__ __forceinline__ bool core_rows(const Layout& L, int i0, int h, int q0
   // LDS (M0) addresses below stay scalar.
   const int l = lane_id(), g = l >> 4, lq = l & 15, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nk = kend;  // a multiple of kKT, at most round_up(n, kKT)
+  // Waves whose queries lie past the written rows (nx is a multiple of 64, the
+  // block's queries of 128) copy and read the last 16 written queries instead.
+  const int qw = min(q0, L.nx - 16);
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
   const bf16* kb[G];
   const bf16* vb[G];
@@ -352,7 +361,7 @@ __device__ __forceinline__ bool core_rows(const Layout& L, int i0, int h, int q0
     kb[r] = L.k + ((int64_t)i * kH + h) * np * kD;
     vb[r] = L.vt + ((int64_t)i * kH + h) * kD * np;
     // Q^T (B operand): query q0 + l%16, head dims 8g .. 8g+7
-    qf[r] = *(const bf16x8*)(L.q + (((int64_t)i * kH + h) * np + q0 + lq) * kD + 8 * g);
+    qf[r] = *(const bf16x8*)(L.q + (((int64_t)i * kH + h) * np + qw + lq) * kD + 8 * g);
   }
 
   // DMA jobs of one stage.  K / V^T: 4 quarters per (row, kind), job
@@ -379,7 +388,7 @@ __device__ __forceinline__ bool core_rows(const Layout& L, int i0, int h, int q0
     }
     kv_lds[u] = (kind == 0 ? kOffK : kOffV) + r * kTileBytes + 1024 * quarter;
   }
-  const bf16* tb_src = L.tb + tb_offset(np, h, q0, 0) + 8 * l;  // + 256 per 16-key block
+  const bf16* tb_src = L.tb + tb_offset(np, h, qw, 0) + 8 * l;  // + 256 per 16-key block
   const int i_mb = min(i0 + (l >> 4), n - 1);
   const float* mb_src = L.mb + (int64_t)i_mb * np + 4 * lq;
   auto dma_stage = [&](int buf, int stage_k0) {
@@ -582,7 +591,7 @@ __device__ __forceinline__ void uniform_rows(const Layout& L, int i0, int h, int
     if (i >= n) break;
     const bf16* vrow = L.vt + (((int64_t)i * kH + h) * kD + d) * np;
     float acc = 0.f;
-    for (int k = 8 * half; k < np; k += 16) {
+    for (int k = 8 * half; k < L.nx; k += 16) {
       const bf16x8 v = gload8(vrow + k);
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc += (float)v[e];
@@ -618,7 +627,7 @@ __global__ __launch_bounds__(kCoreThreads) __attribute__((amdgpu_waves_per_eu(4)
   const int h = col / qtiles, qt = col % qtiles;
   const int t = threadIdx.x, w = t >> 6;
   const int i0 = ig * kRows;
-  const int q0 = qt * kCoreQ + 16 * w;  // this wave's 16 queries (< np: np is a multiple of kCoreQ)
+  const int q0 = qt * kCoreQ + 16 * w;  // this wave's 16 queries
 
   // Row classes from the projection's per-tile key spans: per row, the first
   // masked key and the last open one.  Every wave reduces the same entries
@@ -626,10 +635,10 @@ __global__ __launch_bounds__(kCoreThreads) __attribute__((amdgpu_waves_per_eu(4)
   bool any_mask = false, suffix = true, all_closed = true;
   int kend = 0, mask_from = n;
   {
-    const int l = t & (kWave - 1), tiles = np / kP1;
+    const int l = t & (kWave - 1), tiles = L.nx / kP1;
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
-      const int2* span = L.keyspan + (int64_t)min(i0 + r, n - 1) * tiles;  // rows past n repeat row n-1
+      const int2* span = L.keyspan + (int64_t)min(i0 + r, n - 1) * (np / kP1);  // rows past n repeat row n-1
       int fm = n, lo = -1;
       for (int e = l; e < tiles; e += kWave) {
         const int2 v = span[e];
@@ -798,6 +807,7 @@ Layout make_layout(void* ws, int n) {
   Layout L;
   L.n = n;
   L.np = (int)round_up(n, kPad);
+  L.nx = (int)round_up(n, kP1);
   const int64_t e = qkv_elems(L.np);
   char* p = (char*)ws;
   L.q = (bf16*)p;
@@ -822,7 +832,7 @@ int run(const TIn* x, const float* mask, int n, int starting, float inf, const f
         void* out, int out_mode, const float* row_scale, void* ws, int stages, hipStream_t st) {
   Layout L = make_layout(ws, n);
   if (stages & 1) {
-    const int total = L.np * (L.np / kP1);
+    const int total = L.nx * (L.nx / kP1);
     const int grid = total < 2 * device_cu_count() ? total : 2 * device_cu_count();
     if (starting)
       triattn_proj_kernel<TIn, true><<<dim3(grid), 256, 0, st>>>(x, mask, ln_w, ln_b, eps, w_proj, inf, L);

@@ -14,7 +14,7 @@
 //                     stored), y = p_out(.) * sigmoid(g_out(.)), then write y or
 //                     add it into the fp32 residual stream in place.
 //
-// Operand planes (workspace, bf16, np = round_up(n, 128)):
+// Operand planes (workspace, bf16, np = round_up(n, 64)):
 //   A[c][r][t], B[c][r][t]   outgoing: A=a[r,t], B=b[r,t]; incoming: A=a[t,r], B=b[t,r]
 //   O[c][i][j] = sum_t A[c][i][t] * B[c][j][t]
 // so outgoing O = sum_k a[i,k] b[j,k] and incoming O = sum_k a[k,i] b[k,j]
@@ -28,7 +28,12 @@ using namespace bmx;
 
 namespace {
 
-constexpr int kPlaneTile = 256;        // plane padding granularity (the contraction's 256 x 256 tiles)
+// Plane padding: the projection's tile width and the contraction's stage depth.
+// Padding to the contraction's 256-wide tiles instead cost the projection and
+// the contraction the padded area: at n = 312 (512 instead of 320) 56 and 37 us
+// against 31 and 20, at n = 1134 360 and 533 us against 308 and 449.
+constexpr int kPlaneTile = 64;
+constexpr int kWorkspaceTile = 256;  // padding the workspace query counts (more than the planes use)
 
 // ------------------------------------------------------------------ K1
 // Persistent and weight-stationary: each wave keeps its [p_in; g_in] rows for
@@ -193,7 +198,10 @@ __device__ __forceinline__ void wait_vm() {
 // through the LDS past buffer 0 in two halves of BM / 2 rows; the next tile's
 // first wait then leaves the epilogue's stores in flight (vmcnt counts stores
 // too), so they drain under its stages.
-template <int BM, int BN, int BK, int WM, int WN, int NS>
+// EDGE: np is not a multiple of the tile, so the last row and column of tiles
+// are cut at the planes' end: rows past it are neither copied nor stored, and
+// waves that hold only such rows skip the products.
+template <int BM, int BN, int BK, int WM, int WN, int NS, bool EDGE>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void trimul_contract_kernel(
     const bf16* __restrict__ A, const bf16* __restrict__ B, bf16* __restrict__ O, int np, int tiles_n,
     int tiles_per_ch, int tiles) {
@@ -216,6 +224,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void trimul_contract_ke
   constexpr int kStoresHalf = kHalf * kChunksRow / kThreads;  // 16-byte stores per thread and half
   static_assert(kStoresHalf * kThreads == kHalf * kChunksRow && 2 * kStoresHalf < 64, "uniform epilogue stores");
   static_assert((BM / WM) % 2 == 0, "each half of the rows belongs to whole waves");
+  static_assert(64 % (kRpi * kWaves) == 0, "the rows copied by one instruction of every wave end at 64 rows");
+  static_assert(64 % WM == 0, "edge tiles end on whole waves' rows");
   constexpr int kStageOut = kStage;               // output staging: right after stage buffer 0
   constexpr int kSmem = NS * kStage > kStageOut + kHalf * kORow ? NS * kStage : kStageOut + kHalf * kORow;
   __shared__ __attribute__((aligned(16))) char smem[kSmem];
@@ -224,7 +234,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void trimul_contract_ke
   const int t = threadIdx.x, l = lane_id(), wv = t >> 6;
   const int wm0 = (wv / kWavesN) * WM, wn0 = (wv % kWavesN) * WN;
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
-  auto operands = [&](int T, const bf16*& Ac, const bf16*& Bc, bf16*& Oc) {
+  // mrem, nrem: the tile's rows and columns inside the planes (BM, BN except
+  // at the planes' end; multiples of 64).
+  auto operands = [&](int T, const bf16*& Ac, const bf16*& Bc, bf16*& Oc, int& mrem, int& nrem) {
     const int xcd = T & 7, idx = T >> 3;
     const int c = xcd + 8 * (idx / tiles_per_ch);
     const int tile = idx % tiles_per_ch;
@@ -232,17 +244,21 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void trimul_contract_ke
     Ac = A + c * plane + (int64_t)tm * BM * np;
     Bc = B + c * plane + (int64_t)tn * BN * np;
     Oc = O + c * plane + (int64_t)(tm * BM) * np + tn * BN;
+    mrem = EDGE ? min(BM, np - tm * BM) : BM;
+    nrem = EDGE ? min(BN, np - tn * BN) : BN;
   };
 
   // DMA instruction u of this wave copies tile rows kRpi q .. kRpi q + kRpi - 1
   // (q = wave + kWaves u): lane l -> row kRpi q + l / kCpr, stored chunk
   // l % kCpr holding k-chunk (l % kCpr) ^ ((row / kSwz) % kCpr).
-  auto dma_stage = [&](const bf16* Ac, const bf16* Bc, int k0, int buf) {
+  // Rows past the planes' end are not copied (whole instructions of all waves).
+  auto dma_stage = [&](const bf16* Ac, const bf16* Bc, int mrem, int nrem, int k0, int buf) {
     const unsigned base = lds0 + buf * kStage;
 #pragma unroll
     for (int u = 0; u < kDma; ++u) {
       const bool is_a = u < kDmaA;
       const int q = wv + kWaves * (is_a ? u : u - kDmaA);
+      if (EDGE && kRpi * kWaves * (is_a ? u : u - kDmaA) >= (is_a ? mrem : nrem)) continue;  // block-uniform
       const int row = kRpi * q + l / kCpr, chunk = (l % kCpr) ^ ((row / kSwz) % kCpr);
       const bf16* src = (is_a ? Ac : Bc) + (int64_t)row * np + k0 + 8 * chunk;
       lds_dma16(src, __builtin_amdgcn_readfirstlane(base + (is_a ? 0 : kTileA) + 1024 * q));
@@ -254,53 +270,61 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void trimul_contract_ke
     return *(const bf16x8*)(sb + tile_off + row * (BK * 2) + ((chunk ^ ((row / kSwz) % kCpr)) * 16));
   };
 
-  const int kt_count = np / BK;  // >= 1: np is a multiple of 256
+  const int kt_count = np / BK;  // >= 1: np is a multiple of 64
   const int G = gridDim.x;
   int T = blockIdx.x;
   bool prefetched = false;  // this tile's first stage is in buffer 0, requested before the last epilogue's stores
+  bool stores_left = false;  // ... and those were the whole 2 kStoresHalf stores of a full tile
   while (T < tiles) {  // uniform over the block
     const bf16 *Ac, *Bc;
     bf16* Oc;
-    operands(T, Ac, Bc, Oc);
+    int mrem, nrem;
+    operands(T, Ac, Bc, Oc, mrem, nrem);
+    const bool full = !EDGE || (mrem == BM && nrem == BN);
+    const bool active = !EDGE || (wm0 < mrem && wn0 < nrem);  // wave-uniform
     f32x16 acc[kMi][kNi];
 #pragma unroll
     for (int i = 0; i < kMi; ++i)
 #pragma unroll
       for (int j = 0; j < kNi; ++j) acc[i][j] = zero16();
 
-    if (!prefetched) dma_stage(Ac, Bc, 0, 0);
+    if (!prefetched) dma_stage(Ac, Bc, mrem, nrem, 0, 0);
     for (int kt = 0; kt < kt_count; ++kt) {
       // Stage kt is this wave's oldest outstanding memory operation except
       // for the previous epilogue's stores (first stage of a prefetched
       // tile); the barrier publishes every wave's copy and frees buffer
       // (kt + 1) % 2, read in stage kt - 1.
-      if (kt == 0 && prefetched) wait_vm<2 * kStoresHalf>();
+      if (kt == 0 && stores_left) wait_vm<2 * kStoresHalf>();
       else wait_vm<0>();
       __syncthreads();
-      if (kt + 1 < kt_count) dma_stage(Ac, Bc, (kt + 1) * BK, (kt + 1) & 1);
+      if (kt + 1 < kt_count) dma_stage(Ac, Bc, mrem, nrem, (kt + 1) * BK, (kt + 1) & 1);
       const char* sb = smem + (kt & 1) * kStage;
+      if (active) {
 #pragma unroll
-      for (int ks = 0; ks < BK / 16; ++ks) {
-        bf16x8 af[kMi], bfr[kNi];
+        for (int ks = 0; ks < BK / 16; ++ks) {
+          bf16x8 af[kMi], bfr[kNi];
 #pragma unroll
-        for (int i = 0; i < kMi; ++i) af[i] = sfrag(sb, 0, wm0 + 32 * i, ks);
+          for (int i = 0; i < kMi; ++i) af[i] = sfrag(sb, 0, wm0 + 32 * i, ks);
 #pragma unroll
-        for (int j = 0; j < kNi; ++j) bfr[j] = sfrag(sb, kTileA, wn0 + 32 * j, ks);
+          for (int j = 0; j < kNi; ++j) bfr[j] = sfrag(sb, kTileA, wn0 + 32 * j, ks);
 #pragma unroll
-        for (int i = 0; i < kMi; ++i)
+          for (int i = 0; i < kMi; ++i)
 #pragma unroll
-          for (int j = 0; j < kNi; ++j) acc[i][j] = mfma32(bfr[j], af[i], acc[i][j]);
+            for (int j = 0; j < kNi; ++j) acc[i][j] = mfma32(bfr[j], af[i], acc[i][j]);
+        }
       }
     }
     __syncthreads();  // every wave is done with the stage buffers
 
     int next = T + G;
     prefetched = next < tiles;
+    stores_left = prefetched && full;
     if (prefetched) {  // the next tile's first stage, into buffer 0, ahead of this tile's stores
       const bf16 *An, *Bn;
       bf16* On;
-      operands(next, An, Bn, On);
-      dma_stage(An, Bn, 0, 0);
+      int mn, nn;
+      operands(next, An, Bn, On, mn, nn);
+      dma_stage(An, Bn, mn, nn, 0, 0);
     }
     // acc[i][j] = D[n][m]: lane -> m = wm0 + 32 i + l%32, registers 4q'..4q'+3 ->
     // n = wn0 + 32 j + 8q' + 4(l/32) + 0..3, written as one 8-byte LDS store.
@@ -325,6 +349,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void trimul_contract_ke
       for (int e0 = 0; e0 < kStoresHalf; ++e0) {
         const int e = t + kThreads * e0;
         const int m = e / kChunksRow, ch = e % kChunksRow;
+        if (!full && (h * kHalf + m >= mrem || 8 * ch >= nrem)) continue;
         *(bf16x8*)(Oc + (int64_t)(h * kHalf + m) * np + 8 * ch) = *(const bf16x8*)(smem + kStageOut + m * kORow + 16 * ch);
       }
       __syncthreads();  // the staging rows are free again (and, after the second half, stage buffer 1)
@@ -497,6 +522,25 @@ __global__ __launch_bounds__(256, 2) void trimul_out_kernel(const float* x, cons
 
 inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
+// The contraction in T x T tiles of WM x WN wave tiles.  Two 64-deep stages:
+// 32-deep stages in a 3- or 4-stage ring measured slower (more barriers per
+// k), as did register staging of the operands.  Persistent, `per_cu` blocks
+// per CU (as many as their LDS stages fit), a multiple of 8 blocks so that
+// each keeps one XCD.
+template <int T, int WM, int WN>
+void launch_contract(const bf16* a_pl, const bf16* b_pl, bf16* o_pl, int np, int per_cu, hipStream_t stream) {
+  const int tiles_n = (np + T - 1) / T, tiles_per_ch = tiles_n * tiles_n;
+  const int tiles = kC * tiles_per_ch;
+  const int grid = std::min(tiles, 8 * ((per_cu * device_cu_count() + 7) / 8));
+  const dim3 block((T / WM) * (T / WN) * 64);
+  if (np % T == 0)
+    trimul_contract_kernel<T, T, 64, WM, WN, 2, false>
+        <<<dim3(grid), block, 0, stream>>>(a_pl, b_pl, o_pl, np, tiles_n, tiles_per_ch, tiles);
+  else
+    trimul_contract_kernel<T, T, 64, WM, WN, 2, (T > 64)>
+        <<<dim3(grid), block, 0, stream>>>(a_pl, b_pl, o_pl, np, tiles_n, tiles_per_ch, tiles);
+}
+
 // The three kernels of one module on `workspace` (3 planes of 128 x np x np bf16).
 int launch(const float* x, const float* mask, int ni, int outgoing, const float* norm_in_w, const float* norm_in_b,
            float eps_in, const bf16* w_in, const float* norm_out_w, const float* norm_out_b, float eps_out,
@@ -520,15 +564,20 @@ int launch(const float* x, const float* mask, int ni, int outgoing, const float*
     if (int rc = check_launch("trimul_proj")) return rc;
   }
   if (stages & 2) {
-    // Two 64-deep stages: 32-deep stages in a 3- or 4-stage ring measured
-    // slower (more barriers per k), as did register staging of the operands.
-    constexpr int BM = 256, BN = 256, BK = 64, WM = 64, WN = 128, NS = 2;
-    const int tiles_n = np / BN, tiles_per_ch = (np / BM) * tiles_n;
-    // persistent, one block per CU (its LDS holds two stages), a multiple of 8 so each block keeps one XCD
-    const int tiles = kC * tiles_per_ch;
-    const int grid = std::min(tiles, 8 * ((device_cu_count() + 7) / 8));
-    trimul_contract_kernel<BM, BN, BK, WM, WN, NS>
-        <<<dim3(grid), (BM / WM) * (BN / WN) * 64, 0, stream>>>(a_pl, b_pl, o_pl, np, tiles_n, tiles_per_ch, tiles);
+    // Tile by plane size.  256 x 256 tiles re-read the operands least and are
+    // the fastest where they fill the chip (128 channels x 4 tiles from np = 512
+    // on) and either fit exactly (np = 512: 42 us against 47 in 128-wide tiles,
+    // 1024: 289 against 347) or their cut edge tiles are few (896: 232 against
+    // 245, 1152: 449 against 493).  In between 128-wide tiles win (np = 320: 20
+    // us against 26, 448: 38 and 38, 576: 70 against 84), and 64-wide ones at
+    // np <= 128, where they are the only ones with a block for every CU (117
+    // tokens: 4.7 us against 5.6).
+    if (np > 640 || np == 512)
+      launch_contract<256, 64, 128>(a_pl, b_pl, o_pl, np, 1, stream);
+    else if (np > 128)
+      launch_contract<128, 64, 64>(a_pl, b_pl, o_pl, np, 2, stream);
+    else
+      launch_contract<64, 32, 32>(a_pl, b_pl, o_pl, np, 5, stream);
     if (int rc = check_launch("trimul_contract")) return rc;
   }
   if (stages & 4) {
@@ -613,7 +662,7 @@ extern "C" {
 
 size_t bmx_trimul_workspace_bytes(int64_t n) {
   if (n <= 0) return 0;
-  int64_t np = round_up(n, kPlaneTile);
+  int64_t np = round_up(n, kWorkspaceTile);
   return (size_t)(3 * (int64_t)kC * np * np * (int64_t)sizeof(bf16));
 }
 
