@@ -40,6 +40,10 @@ SIGNATURES = {
     "bmx_swiglu_split3_bf16": (c_int, [_P, c_int64, c_int64, c_int64, _P, _P]),
     "bmx_gated_residual_adaln_split3_bf16": (c_int, [_P, _P, c_int64, _P, _P, _P, _P, c_int64, c_int64, c_int, c_float,
                                                      _P, _P]),
+    "bmx_x3_pack": (c_int, [_P, c_int64, c_int64, c_int64, _P, c_int64, c_int64, _P, _P]),
+    "bmx_token_stack_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int, c_int, c_int64]),
+    "bmx_token_stack_fwd": (c_int, [_P, _P, c_int64, c_int64, c_int, c_int, c_int64, c_int, _P, c_float, _P, _P, c_int64,
+                                    c_int64, c_int64, c_float, _P, _P, c_size_t, _P]),
     "bmx_adaln_strided": (c_int, [_P, _P, _P, c_int64, _P, c_int, c_int64, c_int, c_float, _P]),
     "bmx_gated_residual": (c_int, [_P, _P, c_int64, _P, _P, c_int64, c_int64, _P]),
     "bmx_diffusion_epilogue": (c_int, [c_int, _P, _P, _P, _P, c_int, c_int64, c_int64, _P]),

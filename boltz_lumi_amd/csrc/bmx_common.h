@@ -283,6 +283,26 @@ __device__ __forceinline__ bf16x8 pfrag(const bf16* packed, int cols, int row0, 
   return *(const bf16x8*)(packed + (((int64_t)(row0 >> 5) * (cols >> 4) + ks) * 64 + lane_id()) * 8);
 }
 
+// Packed split operands (linear_x3.hip): fp32 values as bf16 high and low parts
+// in MFMA operand order.  Per 32 rows and 16 columns two contiguous 1 KB runs,
+// high then low, in which lane (row % 32) + 32 * (column % 16 / 8) holds 8
+// columns.  Element index of the high part of (row, col), `ksteps` = columns /
+// 16; the low part is 512 elements on.
+__host__ __device__ __forceinline__ int64_t x3_packed_index(int64_t row, int64_t col, int64_t ksteps) {
+  return ((row >> 5) * ksteps + (col >> 4)) * 1024 + (((row & 31) + 32 * ((col >> 3) & 1)) << 3) + (col & 7);
+}
+__device__ __forceinline__ void x3_packed_store4(bf16* op, int64_t row, int64_t col, int64_t ksteps, f32x4 v) {
+  bf16x4 hi, lo;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    hi[e] = (bf16)v[e];
+    lo[e] = (bf16)(v[e] - (float)hi[e]);
+  }
+  bf16* dst = op + x3_packed_index(row, col, ksteps);
+  *(bf16x4*)dst = hi;
+  *(bf16x4*)(dst + 512) = lo;
+}
+
 }  // namespace bmx
 
 // ---------------------------------------------------------------------------
@@ -294,6 +314,22 @@ int check_launch(const char* what);
 // Compute units of the current device (cached per device; used to size
 // persistent grids).
 int device_cu_count();
+
+// Passes that a token-transformer stack (linear_x3.hip) runs between its
+// linears; op is a packed split operand (x3_packed_index) of `rows` x d.
+int split_packed(const float* x, int64_t rows, int d, bf16* op, hipStream_t stream);
+int layernorm_packed(const float* x, int64_t rows, int d, float eps, bf16* op, hipStream_t stream);
+int adaln_packed(const float* a, const float* scale, const float* shift, int64_t ldm, int64_t rows, int d, float eps,
+                 bf16* op, hipStream_t stream);
+int gated_residual_adaln_packed(const float* a, const float* g, int64_t ldg, const float* c, float* out,
+                                const float* scale, const float* shift, int64_t ldm, int64_t rows, int d, float eps,
+                                bf16* op, hipStream_t stream);
+// Attention of one layer from proj = [q | k | v | g] rows (4 H D columns), its
+// gated output as the packed operand op.
+int token_attention_packed(const float* proj, int64_t batch, int64_t n, int heads, int head_dim, const float* bias,
+                           int64_t sbias, int64_t bias_div, const float* mask, int64_t smask, float inf, bf16* op,
+                           void* ws, hipStream_t stream);
+size_t token_attention_workspace(int64_t batch, int64_t n, int heads, int head_dim);
 }  // namespace bmx
 
 #define BMX_OK 0

@@ -124,7 +124,7 @@ __global__ __launch_bounds__(256) void seq_attention_kernel(const float* __restr
                                                             const float* __restrict__ mask,
                                                             const float* __restrict__ g, SeqAttnShape sh, int heads,
                                                             float inf, float rscale, int vec,
-                                                            float* __restrict__ out) {
+                                                            float* __restrict__ out, bf16* __restrict__ packed) {
   constexpr int KS = D / 4;          // QK^T MFMA steps
   constexpr int DT = (D + 15) / 16;  // O^T d tiles
   static_assert(D % 4 == 0, "head dim");
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void seq_attention_kernel(const float* __restr
     v += b * sh.sk;
     bias += (b / sh.bdiv) * sh.sbg + (b % sh.bwin) * sh.sbias;
     mask += b * sh.smask;
-    out += b * nq * HD;
+    if (out) out += b * nq * HD;
     if (sh.nw > 0) {
       const int t0 = (int)(b % sh.nw) * sh.wq + sh.koff;
       klo = max(0, -t0);
@@ -258,14 +258,22 @@ __global__ __launch_bounds__(256) void seq_attention_kernel(const float* __restr
 #pragma unroll
       for (int u = 0; u < kAttnWaves; ++u) acc += wt[u] * part_o[u][d][qi];
       const float gate = sigmoid_f(g[(int64_t)i * ldq + h * D + d]);
-      out[(int64_t)i * HD + h * D + d] = gate * (acc / ll);
+      const float y = gate * (acc / ll);
+      if (packed) {  // the row as a packed split operand
+        bf16* dst = packed + x3_packed_index((int64_t)blockIdx.z * nq + i, h * D + d, HD >> 4);
+        const bf16 hi = (bf16)y;
+        dst[0] = hi;
+        dst[512] = (bf16)(y - (float)hi);
+      } else {
+        out[(int64_t)i * HD + h * D + d] = y;
+      }
     }
   }
 }
 
 int launch_seq_attention(const char* name, const float* q, const float* k, const float* v, const float* bias,
                          const float* mask, const float* g, int64_t batch, SeqAttnShape sh, int heads,
-                         int head_dim, float inf, float* out, hipStream_t stream) {
+                         int head_dim, float inf, float* out, hipStream_t stream, bf16* packed = nullptr) {
   if (sh.sbq == 0) {  // dense [heads][nq][nk] bias elements
     sh.sbh = (int64_t)sh.nq * sh.nk;
     sh.sbq = sh.nk;
@@ -280,11 +288,14 @@ int launch_seq_attention(const char* name, const float* q, const float* k, const
   const dim3 grid((unsigned)((sh.nq + kAttnQ - 1) / kAttnQ), (unsigned)heads, (unsigned)batch);
   const float rscale = 1.f / sqrtf((float)head_dim);
 #define SEQ_ATTN(DIM, TILES) \
-  seq_attention_kernel<DIM, TILES><<<grid, 256, 0, stream>>>(q, k, v, bias, mask, g, sh, heads, inf, rscale, vec, out)
+  seq_attention_kernel<DIM, TILES><<<grid, 256, 0, stream>>>(q, k, v, bias, mask, g, sh, heads, inf, rscale, vec, out, \
+                                                           packed)
   const bool short_keys = sh.nk <= kAttnWaves * 32;
-  if (head_dim == 24) SEQ_ATTN(24, 4);
+  if (head_dim == 24 && short_keys) SEQ_ATTN(24, 2);
+  else if (head_dim == 24) SEQ_ATTN(24, 4);
   else if (head_dim == 32 && short_keys) SEQ_ATTN(32, 2);
   else if (head_dim == 32) SEQ_ATTN(32, 4);
+  else if (short_keys) SEQ_ATTN(48, 2);
   else SEQ_ATTN(48, 4);
 #undef SEQ_ATTN
   return check_launch(name);
@@ -433,7 +444,8 @@ __global__ __launch_bounds__(256) void seq_attention_x3_kernel(const float* __re
                                                                const float* __restrict__ bias,
                                                                const float* __restrict__ g, SeqAttnShape sh, int heads,
                                                                int64_t batch, float rscale, bool vec,
-                                                               float* __restrict__ out, bf16* __restrict__ op) {
+                                                               float* __restrict__ out, bf16* __restrict__ op,
+                                                               bool packed) {
   constexpr bool T16 = D % 32 == 16;             // the last 16 dims on a K = 16 MFMA
   constexpr int DK = T16 ? D / 32 : (D + 31) / 32;  // QK^T k steps of 32 dims
   constexpr int DT = (D + 15) / 16;              // O^T d tiles
@@ -627,7 +639,9 @@ __global__ __launch_bounds__(256) void seq_attention_x3_kernel(const float* __re
         f32x4 r;
 #pragma unroll
         for (int e = 0; e < 4; ++e) r[e] = sigmoid_f(gv[e]) * (o[dt][e] * inv);
-        if (orow) {
+        if (packed) {
+          x3_packed_store4(op, (int64_t)b * nq + i, h * D + d0, HD >> 4, r);
+        } else if (orow) {
           bf16x4 hi, lo;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -642,7 +656,7 @@ __global__ __launch_bounds__(256) void seq_attention_x3_kernel(const float* __re
         }
       }
     }
-    if (orow && h == 0) {  // lanes gi = 0..3 write 16 tail columns each
+    if (orow && !packed && h == 0) {  // lanes gi = 0..3 write 16 tail columns each
       bf16x8 t = {};
       if (gi == 0) t[0] = t[1] = (bf16)1.f;
       *(bf16x8*)(orow + 3 * HD + 16 * gi) = t;
@@ -659,7 +673,8 @@ size_t x3_workspace_bytes(int64_t batch, int64_t nk, int heads, int head_dim) {
 
 int launch_seq_attention_x3(const char* name, const float* q, const float* k, const float* v, const float* bias,
                             const float* mask, const float* g, int64_t batch, const SeqAttnShape& sh, int heads,
-                            int head_dim, float inf, float* out, bf16* op, void* ws, hipStream_t stream) {
+                            int head_dim, float inf, float* out, bf16* op, void* ws, hipStream_t stream,
+                            bool packed = false) {
   const int64_t hd = (int64_t)heads * head_dim, nkp = x3_nkp(sh.nk);
   const size_t tile = ((size_t)(batch * hd * nkp) * sizeof(bf16) + 255) / 256 * 256;
   bf16* kh = (bf16*)ws;
@@ -686,7 +701,7 @@ int launch_seq_attention_x3(const char* name, const float* q, const float* k, co
   const float rscale = 1.f / sqrtf((float)head_dim);
 #define SEQ_ATTN_X3(DIM)                                                                                       \
   seq_attention_x3_kernel<DIM><<<grid, 256, 0, stream>>>(q, kh, kl, vth, vtl, mterm, bias, g, sh, heads, batch, \
-                                                         rscale, vec, out, op)
+                                                         rscale, vec, out, op, packed)
   if (head_dim == 24) SEQ_ATTN_X3(24);
   else if (head_dim == 32) SEQ_ATTN_X3(32);
   else SEQ_ATTN_X3(48);
@@ -694,7 +709,33 @@ int launch_seq_attention_x3(const char* name, const float* q, const float* k, co
   return check_launch(name);
 }
 
+// From this many keys on the split-bf16 kernel runs the token attention (as
+// the Python wrapper chooses), below it the fp32 one: the pre-pass costs more
+// than the shorter products save.
+constexpr int64_t kX3MinKeys = 256;
+
 }  // namespace
+
+namespace bmx {
+
+size_t token_attention_workspace(int64_t batch, int64_t n, int heads, int head_dim) {
+  return n >= kX3MinKeys ? x3_workspace_bytes(batch, n, heads, head_dim) : 0;
+}
+
+int token_attention_packed(const float* proj, int64_t batch, int64_t n, int heads, int head_dim, const float* bias,
+                           int64_t sbias, int64_t bias_div, const float* mask, int64_t smask, float inf, bf16* op,
+                           void* ws, hipStream_t stream) {
+  const int64_t hd = (int64_t)heads * head_dim, ld = 4 * hd;
+  const SeqAttnShape sh{(int)n, (int)n, (int)bias_div, ld, ld, n * ld, n * ld, sbias, smask};
+  const float *q = proj, *k = proj + hd, *v = proj + 2 * hd, *g = proj + 3 * hd;
+  if (n >= kX3MinKeys)
+    return launch_seq_attention_x3("token_attention", q, k, v, bias, mask, g, batch, sh, heads, head_dim, inf, nullptr,
+                                   op, ws, stream, true);
+  return launch_seq_attention("token_attention", q, k, v, bias, mask, g, batch, sh, heads, head_dim, inf, nullptr,
+                              stream, op);
+}
+
+}  // namespace bmx
 
 extern "C" {
 

@@ -23,6 +23,9 @@
 //  bmx_gated_residual_adaln_split3_bf16  c + sigmoid(g) * a -> out, and the AdaLN
 //                             operand of that new row
 //
+// The same writers, with the operand in packed MFMA order instead
+// (x3_packed_index), feed the token transformer's own linears (linear_x3.hip).
+//
 // None has a reference counterpart: the reference leaves these fp32 linears
 // and the passes in front of them to torch (diffusion.py:52-68,
 // pair_bias.py:15-36).  One wave per row, four rows per 256-thread block.
@@ -55,15 +58,35 @@ __device__ __forceinline__ void put_tail(bf16* row, int64_t k, int lane) {
   }
 }
 
+// The operand row `row` of `rows x k` values: [hi | hi | lo | tail] rows, or the
+// packed order.
+template <bool PACKED>
+struct OperandRow {
+  bf16* op;
+  int64_t row, k;
+  __device__ __forceinline__ OperandRow(bf16* out, int64_t row, int64_t k)
+      : op(PACKED ? out : out + row * (3 * k + kTail)), row(row), k(k) {}
+  __device__ __forceinline__ void put(int64_t col, f32x4 v) const {
+    if constexpr (PACKED)
+      x3_packed_store4(op, row, col, k >> 4, v);
+    else
+      put_split(op, k, col, v);
+  }
+  __device__ __forceinline__ void tail(int lane) const {
+    if constexpr (!PACKED) put_tail(op, k, lane);
+  }
+};
+
+template <bool PACKED>
 __global__ __launch_bounds__(256) void split3_kernel(const float* __restrict__ x, int64_t ldx, bf16* __restrict__ out,
                                                      int64_t rows, int64_t k) {
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int lane = threadIdx.x & 63;
   const float* xr = x + row * ldx;
-  bf16* o = out + row * (3 * k + kTail);
-  for (int64_t c = 4 * lane; c < k; c += 4 * kWave) put_split(o, k, c, load4(xr + c));
-  put_tail(o, k, lane);
+  const OperandRow<PACKED> o(out, row, k);
+  for (int64_t c = 4 * lane; c < k; c += 4 * kWave) o.put(c, load4(xr + c));
+  o.tail(lane);
 }
 
 // Row statistics of LayerNorm over d values held as float4 chunks
@@ -92,6 +115,7 @@ __device__ __forceinline__ RowNorm row_norm(const f32x4 (&v)[kRowChunks], int la
 
 // tn > 0: the rows of x are the pairs of a tn x tn frame read transposed
 // (operand row i tn + j is x row j tn + i).
+template <bool PACKED>
 __global__ __launch_bounds__(256) void layernorm_split3_kernel(const float* __restrict__ x, int64_t ldx,
                                                                bf16* __restrict__ out, int64_t rows, int d,
                                                                float eps, int64_t tn) {
@@ -104,15 +128,16 @@ __global__ __launch_bounds__(256) void layernorm_split3_kernel(const float* __re
 #pragma unroll
   for (int u = 0; u < kRowChunks; ++u) v[u] = load4(xr + 4 * min(lane + kWave * u, chunks - 1));
   const RowNorm n = row_norm(v, lane, chunks, d, eps);
-  bf16* o = out + row * (3 * (int64_t)d + kTail);
+  const OperandRow<PACKED> o(out, row, d);
 #pragma unroll
   for (int u = 0; u < kRowChunks; ++u)
-    if (lane + kWave * u < chunks) put_split(o, d, 4 * (lane + kWave * u), (v[u] - n.mean) * n.inv);
-  put_tail(o, d, lane);
+    if (lane + kWave * u < chunks) o.put(4 * (lane + kWave * u), (v[u] - n.mean) * n.inv);
+  o.tail(lane);
 }
 
 // sigmoid(scale) * LN(a) + shift as bmx_adaln rounds it (the product and the
 // sum separately), scale and shift rows at stride ldm.
+template <bool PACKED>
 __global__ __launch_bounds__(256) void adaln_split3_kernel(const float* __restrict__ a, const float* __restrict__ scale,
                                                            const float* __restrict__ shift, int64_t ldm,
                                                            bf16* __restrict__ out, int64_t rows, int d, float eps) {
@@ -129,7 +154,7 @@ __global__ __launch_bounds__(256) void adaln_split3_kernel(const float* __restri
     sh[u] = load4(shift + row * ldm + c);
   }
   const RowNorm n = row_norm(v, lane, chunks, d, eps);
-  bf16* o = out + row * (3 * (int64_t)d + kTail);
+  const OperandRow<PACKED> o(out, row, d);
 #pragma unroll
   for (int u = 0; u < kRowChunks; ++u) {
     if (lane + kWave * u < chunks) {
@@ -140,16 +165,17 @@ __global__ __launch_bounds__(256) void adaln_split3_kernel(const float* __restri
         const float prod = sigmoid_f(sc[u][e]) * an;
         r[e] = prod + sh[u][e];
       }
-      put_split(o, d, 4 * (lane + kWave * u), r);
+      o.put(4 * (lane + kWave * u), r);
     }
   }
-  put_tail(o, d, lane);
+  o.tail(lane);
 }
 
 // The residual update of a diffusion layer and the next AdaLN in one pass:
 // r = c + sigmoid(g) * a (the MODULATION epilogue; g and the modulation rows at
 // strides ldg / ldm) is written to out (which may alias c), then the operand
 // row of sigmoid(scale) * LN(r) + shift, rounded as bmx_adaln_split3_bf16.
+template <bool PACKED>
 __global__ __launch_bounds__(256) void gated_residual_adaln_split3_kernel(
     const float* __restrict__ a, const float* __restrict__ g, int64_t ldg, const float* c, float* out,
     const float* __restrict__ scale, const float* __restrict__ shift, int64_t ldm, bf16* __restrict__ op,
@@ -175,7 +201,7 @@ __global__ __launch_bounds__(256) void gated_residual_adaln_split3_kernel(
   for (int u = 0; u < kRowChunks; ++u)
     if (lane + kWave * u < chunks) store4(out + row * d + 4 * (lane + kWave * u), v[u]);
   const RowNorm n = row_norm(v, lane, chunks, d, eps);
-  bf16* o = op + row * (3 * (int64_t)d + kTail);
+  const OperandRow<PACKED> o(op, row, d);
 #pragma unroll
   for (int u = 0; u < kRowChunks; ++u) {
     if (lane + kWave * u < chunks) {
@@ -186,10 +212,10 @@ __global__ __launch_bounds__(256) void gated_residual_adaln_split3_kernel(
         const float prod = sigmoid_f(sc[u][e]) * an;
         r[e] = prod + sh[u][e];
       }
-      put_split(o, d, 4 * (lane + kWave * u), r);
+      o.put(4 * (lane + kWave * u), r);
     }
   }
-  put_tail(o, d, lane);
+  o.tail(lane);
 }
 
 // Row r of u holds [x | g | b] (3 cols values at stride ldu): the swish gate's
@@ -221,6 +247,34 @@ inline unsigned row_blocks(int64_t rows) { return (unsigned)((rows + 3) / 4); }
 
 }  // namespace
 
+namespace bmx {
+
+int split_packed(const float* x, int64_t rows, int d, bf16* op, hipStream_t stream) {
+  split3_kernel<true><<<row_blocks(rows), 256, 0, stream>>>(x, d, op, rows, d);
+  return check_launch("split_packed");
+}
+
+int layernorm_packed(const float* x, int64_t rows, int d, float eps, bf16* op, hipStream_t stream) {
+  layernorm_split3_kernel<true><<<row_blocks(rows), 256, 0, stream>>>(x, d, op, rows, d, eps, 0);
+  return check_launch("layernorm_packed");
+}
+
+int adaln_packed(const float* a, const float* scale, const float* shift, int64_t ldm, int64_t rows, int d, float eps,
+                 bf16* op, hipStream_t stream) {
+  adaln_split3_kernel<true><<<row_blocks(rows), 256, 0, stream>>>(a, scale, shift, ldm, op, rows, d, eps);
+  return check_launch("adaln_packed");
+}
+
+int gated_residual_adaln_packed(const float* a, const float* g, int64_t ldg, const float* c, float* out,
+                                const float* scale, const float* shift, int64_t ldm, int64_t rows, int d, float eps,
+                                bf16* op, hipStream_t stream) {
+  gated_residual_adaln_split3_kernel<true>
+      <<<row_blocks(rows), 256, 0, stream>>>(a, g, ldg, c, out, scale, shift, ldm, op, rows, d, eps);
+  return check_launch("gated_residual_adaln_packed");
+}
+
+}  // namespace bmx
+
 extern "C" {
 
 int bmx_split3_bf16(const float* x, int64_t rows, int64_t k, int64_t ldx, void* out, hipStream_t stream) {
@@ -231,7 +285,7 @@ int bmx_split3_bf16(const float* x, int64_t rows, int64_t k, int64_t ldx, void* 
   BMX_REQUIRE(x && out, "bmx_split3_bf16: null pointer");
   BMX_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)out % 8 == 0,
               "bmx_split3_bf16: x must be 16-byte and out 8-byte aligned");
-  split3_kernel<<<row_blocks(rows), 256, 0, stream>>>(x, ldx, (bf16*)out, rows, k);
+  split3_kernel<false><<<row_blocks(rows), 256, 0, stream>>>(x, ldx, (bf16*)out, rows, k);
   return check_launch("bmx_split3_bf16");
 }
 
@@ -245,7 +299,7 @@ int bmx_layernorm_split3_bf16(const float* x, int64_t rows, int dim, int64_t ldx
   BMX_REQUIRE(x && out, "bmx_layernorm_split3_bf16: null pointer");
   BMX_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)out % 8 == 0,
               "bmx_layernorm_split3_bf16: x must be 16-byte and out 8-byte aligned");
-  layernorm_split3_kernel<<<row_blocks(rows), 256, 0, stream>>>(x, ldx, (bf16*)out, rows, dim, eps, 0);
+  layernorm_split3_kernel<false><<<row_blocks(rows), 256, 0, stream>>>(x, ldx, (bf16*)out, rows, dim, eps, 0);
   return check_launch("bmx_layernorm_split3_bf16");
 }
 
@@ -259,7 +313,7 @@ int bmx_layernorm_split3_t_bf16(const float* x, int64_t n, int dim, int64_t ldx,
   BMX_REQUIRE(x && out, "bmx_layernorm_split3_t_bf16: null pointer");
   BMX_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)out % 8 == 0,
               "bmx_layernorm_split3_t_bf16: x must be 16-byte and out 8-byte aligned");
-  layernorm_split3_kernel<<<row_blocks(n * n), 256, 0, stream>>>(x, ldx, (bf16*)out, n * n, dim, eps, n);
+  layernorm_split3_kernel<false><<<row_blocks(n * n), 256, 0, stream>>>(x, ldx, (bf16*)out, n * n, dim, eps, n);
   return check_launch("bmx_layernorm_split3_t_bf16");
 }
 
@@ -274,7 +328,7 @@ int bmx_adaln_split3_bf16(const float* a, const float* scale, const float* shift
   BMX_REQUIRE(a && scale && shift && out, "bmx_adaln_split3_bf16: null pointer");
   BMX_REQUIRE(((uintptr_t)a | (uintptr_t)scale | (uintptr_t)shift) % 16 == 0 && (uintptr_t)out % 8 == 0,
               "bmx_adaln_split3_bf16: a, scale, shift must be 16-byte and out 8-byte aligned");
-  adaln_split3_kernel<<<row_blocks(rows), 256, 0, stream>>>(a, scale, shift, ld_mod, (bf16*)out, rows, dim, eps);
+  adaln_split3_kernel<false><<<row_blocks(rows), 256, 0, stream>>>(a, scale, shift, ld_mod, (bf16*)out, rows, dim, eps);
   return check_launch("bmx_adaln_split3_bf16");
 }
 
@@ -293,7 +347,7 @@ int bmx_gated_residual_adaln_split3_bf16(const float* a, const float* gate, int6
                       16 == 0 &&
                   (uintptr_t)op % 8 == 0,
               "bmx_gated_residual_adaln_split3_bf16: fp32 operands must be 16-byte and op 8-byte aligned");
-  gated_residual_adaln_split3_kernel<<<row_blocks(rows), 256, 0, stream>>>(a, gate, ld_gate, c, out, scale, shift,
+  gated_residual_adaln_split3_kernel<false><<<row_blocks(rows), 256, 0, stream>>>(a, gate, ld_gate, c, out, scale, shift,
                                                                            ld_mod, (bf16*)op, rows, dim, eps);
   return check_launch("bmx_gated_residual_adaln_split3_bf16");
 }

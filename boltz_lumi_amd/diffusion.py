@@ -354,6 +354,113 @@ def layer_forward(self, a, s, bias=None, mask=None, to_keys=None, multiplicity=1
     return _layer(self, a, s, bias, mask, to_keys, multiplicity, None)
 
 
+# Up to this many rows (samples x tokens) the token stack runs as one native
+# call on its own few-row linears (bmx_token_stack_fwd); above, per layer on the
+# library's split-bf16 GEMMs (linear_x3.hip holds both sides' times).
+TOKEN_STACK_MAX_ROWS = 1024
+
+
+def _stack_pack(layer, d, inner):
+    """One layer's packed weights and fp32 biases in the order of
+    ``bmx_token_stack_fwd`` (pair bias last, left to the caller), as
+    (tensors, eps of the two a_norms)."""
+    att, tr = layer.pair_bias_attn, layer.transition
+    dev = att.proj_q.weight.device
+
+    def pack(rows, k, *parts):  # parts: (tile0, tile stride, weight, column scale)
+        out = torch.empty(rows * k * 2, device=dev, dtype=torch.bfloat16)
+        for tile0, stride, w, scale in parts:
+            ops.x3_pack(out, tile0, w, stride, scale)
+        return out
+
+    def biases(pairs):  # concatenated biases of (linear, bias or None); None when there is none
+        if all(b is None for _, b in pairs):
+            return None
+        return torch.cat([b.detach().float() if b is not None
+                          else lin.weight.new_zeros(lin.out_features, dtype=torch.float32) for lin, b in pairs])
+
+    def cond(lin, sn):  # s_scale / s_bias of an AdaLN: the s_norm weight is the column scale, its bias folds into b
+        b = lin.bias
+        if sn.bias is not None:
+            fold = lin.weight.detach().float() @ sn.bias.detach().float()
+            b = fold if b is None else b.detach().float() + fold
+        return lin, b
+
+    t = d // 32
+    ads = (layer.adaln, tr.adaln)
+    gates = _gate_linears(layer)
+    parts, pairs = [], []
+    for i, ad in enumerate(ads):
+        for j, lin in enumerate((ad.s_scale, ad.s_bias)):
+            parts.append(((2 * i + j) * t, 1, lin.weight, ad.s_norm.weight))
+            pairs.append(cond(lin, ad.s_norm))
+    for i, lin in enumerate(gates):
+        parts.append(((4 + i) * t, 1, lin.weight, None))
+        pairs.append((lin, lin.bias))
+    qkvg = (att.proj_q, att.proj_k, att.proj_v, att.proj_g)
+    sw, ab, down = tr.swish_gate[0], tr.a_to_b, tr.b_to_a
+    up_bias = None
+    if sw.bias is not None or ab.bias is not None:
+        up_bias = biases([(sw, sw.bias), (ab, ab.bias)])
+    return (pack(6 * d, d, *parts), biases(pairs),
+            pack(4 * d, d, *[(i * t, 1, lin.weight, None) for i, lin in enumerate(qkvg)]),
+            biases([(lin, lin.bias) for lin in qkvg]),
+            pack(d, d, (0, 1, att.proj_o.weight, None)), biases([(att.proj_o, att.proj_o.bias)]),
+            pack(3 * inner, d, (0, 3, sw.weight[:inner], None), (1, 3, sw.weight[inner:], None),
+                 (2, 3, ab.weight, None)), up_bias,
+            pack(d, inner, (0, 1, down.weight, None)), biases([(down, down.bias)]))
+
+
+def _stack_sources(layer):
+    att, tr = layer.pair_bias_attn, layer.transition
+    lins = (att.proj_q, att.proj_k, att.proj_v, att.proj_g, att.proj_o, tr.swish_gate[0], tr.a_to_b,
+            tr.b_to_a) + _gate_linears(layer)
+    return _mods_sources(layer) + tuple(p for lin in lins for p in (lin.weight, lin.bias) if p is not None)
+
+
+def _native_stack(layers, a, s, biases, mask, multiplicity):
+    """The whole stack as one ``bmx_token_stack_fwd`` call, or None where it
+    does not apply: layers whose chain already runs on split operands
+    (``_with_side_ok``, ``_operand_path``) with plain proj_o and Identity
+    post_lnorm, one shape, one s_norm eps and one attention inf throughout, and
+    at most ``TOKEN_STACK_MAX_ROWS`` rows.  ``biases``: every layer's pair bias
+    as its attention's proj_z takes it."""
+    b, n, d = a.shape
+    first = layers[0].pair_bias_attn
+    heads, inner = first.num_heads, layers[0].transition.a_to_b.out_features
+    eps_s, inf = layers[0].adaln.s_norm.eps, first.inf
+    if d % 32 or inner % 32 or first.c_s != d:
+        return None
+    for layer in layers:
+        att, tr = layer.pair_bias_attn, layer.transition
+        if not (type(layer.post_lnorm) is torch.nn.Identity and _untouched(layer.post_lnorm) and _untouched(att.proj_o)
+                and att.num_heads == heads and att.c_s == d and att.inf == inf and layer.adaln.s_norm.eps == eps_s
+                and tr.a_to_b.out_features == inner and tuple(tr.swish_gate[0].weight.shape) == (2 * inner, d)
+                and tuple(tr.b_to_a.weight.shape) == (d, inner)):
+            return None
+    m = mask.float()
+    if m.dim() != 2 or m.shape[1] != n or m.shape[0] not in (1, b):
+        return None
+    if m.stride(1) != 1:
+        m = m.contiguous()
+    params, keep, eps, sbias = [], [m], [], None
+    for layer, z in zip(layers, biases):
+        att = layer.pair_bias_attn
+        zb = att.proj_z(z)
+        if not (zb.dtype == torch.float32 and zb.dim() == 4 and zb.shape[0] * multiplicity == b
+                and tuple(zb.shape[1:]) == (heads, n, n) and zb.device == a.device and zb[0].is_contiguous()):
+            return None
+        stride = zb.stride(0) if zb.shape[0] > 1 else 0
+        if sbias is not None and stride != sbias:
+            return None
+        sbias = stride
+        pack = ops.cached_value(layer, "token_stack", _stack_sources(layer), lambda: _stack_pack(layer, d, inner))
+        keep += [zb, pack]
+        params += [0 if t is None else t.data_ptr() for t in pack] + [zb.data_ptr()]
+        eps += [layer.adaln.a_norm.eps, layer.transition.adaln.a_norm.eps]
+    return ops.token_stack(a, s, params, eps, eps_s, heads, inner, m, sbias, multiplicity, inf)
+
+
 def stack_forward(self, a, s, bias=None, mask=None, to_keys=None, multiplicity=1):
     """Drop-in for ``DiffusionTransformer.forward`` (upstream transformersv2):
     the same per-layer loop, with the layers' operands of s built once per
@@ -370,6 +477,11 @@ def stack_forward(self, a, s, bias=None, mask=None, to_keys=None, multiplicity=1
     # consecutive layers on the operand path chain their boundary passes: layer
     # i's last residual update also writes layer i + 1's attention operand
     chain = [_with_side_ok(l, a, s) and _operand_path(l, side, to_keys) for l in layers]
+    if (all(chain) and mask is not None and a.dim() == 3 and 0 < a.shape[0] * a.shape[1] <= TOKEN_STACK_MAX_ROWS
+            and getattr(self, "pair_bias_attn", True)):
+        out = _native_stack(layers, a, s, [bias[:, :, :, i] for i in range(len(layers))], mask, multiplicity)
+        if out is not None:
+            return out
     carry = None
     for i, layer in enumerate(layers):
         bias_l = bias[:, :, :, i] if getattr(self, "pair_bias_attn", True) else None

@@ -17,6 +17,7 @@ raises.
 
 from __future__ import annotations
 
+import ctypes
 import os
 
 import torch
@@ -54,6 +55,23 @@ def _cuda(*tensors: torch.Tensor) -> None:
 
 def _inference_only() -> None:
     _check(not torch.is_grad_enabled(), "Inference only")
+
+
+def cached_value(module, name: str, sources, build):
+    """``build()`` cached on ``module`` under ``name`` by the rule of
+    ``cached_weight`` (any value, e.g. several packed weights at once)."""
+    if any(p.is_inference() for p in sources):
+        with torch.no_grad():
+            return build()
+    key = tuple((id(p), p._version, p.data_ptr(), p.device, p.dtype) for p in sources)
+    cache = module.__dict__.setdefault("_bmx_weight_cache", {})
+    hit = cache.get(name)
+    if hit is None or hit[0] != key:
+        with torch.no_grad():
+            value = build()
+        hit = (key, value)
+        cache[name] = hit
+    return hit[1]
 
 
 def cached_weight(module, name: str, sources, build):
@@ -461,6 +479,16 @@ def linear_x3(x, linear):
     w = x3_weight(linear, "x3", (linear.weight,), (linear.bias,))
     y = mm_x3(x.reshape(-1, k), w)
     return y.view(x.shape[:-1] + (w.shape[0],))
+
+
+def x3_pack(out, tile0, w, tile_stride=1, col_scale=None):
+    """Weight rows ``w`` [N, K] (times ``col_scale`` [K] per column) into the
+    packed split operand ``out`` (``bmx_x3_pack``): 32-row tile t at tile
+    ``tile0 + t * tile_stride``."""
+    w = _f32(w)
+    scale = None if col_scale is None else _f32(col_scale)
+    N.call("bmx_x3_pack", w.data_ptr(), w.shape[0], w.shape[1], w.stride(0), None if scale is None else scale.data_ptr(),
+           tile0, tile_stride, out.data_ptr(), _stream(w))
 
 
 MODULATION, GATE, GATED_SWIGLU = 0, 1, 3
@@ -974,6 +1002,30 @@ def seq_attention_windowed(q, k, v, bias, mask, g, inf, *, windows, key_offset, 
                mask.data_ptr(), g.data_ptr(), e, w, nk, q.stride(1), k.stride(0), windows, key_offset, bias_group,
                bias.stride(0), bias.stride(1), bias.stride(4), bias.stride(2), bias.stride(3), heads, width // heads,
                float(inf), out.data_ptr(), _stream(q))
+    return out
+
+
+def token_stack(a, s, params, eps, eps_s, heads, inner, mask, sbias, bias_div, inf):
+    """A stack of diffusion transformer layers on at most 1024 rows as one
+    native call (``bmx_token_stack_fwd``): a, s [B, N, d] fp32, ``params`` the
+    11 device addresses per layer and ``eps`` the 2 a_norm eps per layer in its
+    order, mask [1 or B, N] with unit stride, ``sbias`` the pair bias's stride
+    per structure of ``bias_div`` samples."""
+    _cuda(a, s, mask)
+    _check(a.shape == s.shape and a.dim() == 3 and a.dtype == s.dtype == mask.dtype == torch.float32
+           and a.is_contiguous() and s.is_contiguous(), "expected contiguous fp32 a and s [B, N, d]")
+    b, n, d = a.shape
+    layers = len(eps) // 2
+    _check(len(params) == 11 * layers and len(eps) == 2 * layers, "expected 11 addresses and 2 eps per layer")
+    _check(mask.dim() == 2 and mask.shape[1] == n and mask.shape[0] in (1, b) and mask.stride(1) == 1,
+           "expected an fp32 [B or 1, N] mask")
+    out = torch.empty_like(a)
+    nbytes = N.lib().bmx_token_stack_workspace_bytes(b, n, heads, d // heads, inner)
+    ws = _workspace(nbytes, a.device)
+    N.call("bmx_token_stack_fwd", a.data_ptr(), s.data_ptr(), b, n, heads, d // heads, inner, layers,
+           (ctypes.c_void_p * len(params))(*params), float(eps_s), (ctypes.c_float * len(eps))(*eps), mask.data_ptr(),
+           mask.stride(0) if mask.shape[0] > 1 else 0, sbias, bias_div, float(inf), out.data_ptr(), ws.data_ptr(),
+           ws.numel(), _stream(a))
     return out
 
 

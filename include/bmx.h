@@ -141,6 +141,35 @@ int bmx_gated_residual_adaln_split3_bf16(const float* a, const float* gate, int6
                                          float* out, const float* scale, const float* shift, int64_t ld_mod,
                                          int64_t rows, int dim, float eps, void* op, bmx_stream_t stream);
 
+/* fp32 weight rows (times col_scale per column, or NULL) as a packed split-bf16 operand:
+ * per 32 rows and 16 columns two contiguous 1 KB runs, bf16 high then low parts, in MFMA
+ * operand order (lane (row % 32) + 32 (column % 16 / 8) holds 8 columns).  32-row tile t goes
+ * to packed tile tile0 + t * tile_stride, so that several weights interleave in one operand.
+ * rows a multiple of 32, k a multiple of 16; 4 * k bytes per row.  No reference kernel: the
+ * reference leaves these linears to torch (diffusion.py:52-68, pair_bias.py:15-36). */
+int bmx_x3_pack(const float* w, int64_t rows, int64_t k, int64_t ldw, const float* col_scale, int64_t tile0,
+                int64_t tile_stride, void* out, bmx_stream_t stream);
+
+/* A stack of diffusion transformer layers for few rows (batch * n <= 1024): transformersv2
+ * DiffusionTransformer, whose AdaLN, attention and conditioned transition the reference patches
+ * one by one (diffusion.py:52-68, pair_bias.py:15-36).  a, s, out: fp32 [batch * n, d], d =
+ * heads * head_dim; out may not alias a or s.  params: 11 device pointers per layer (host array):
+ *   0 w_cond   [6 d, d] packed: both AdaLNs' s_scale and s_bias with the s_norm weight as
+ *              col_scale (attention's, then the transition's), then both output gates
+ *   1 b_cond   [6 d] or NULL
+ *   2 w_qkvg   [4 d, d], 3 its bias; 4 w_o [d, d], 5 its bias
+ *   6 w_up     [3 inner, d]: 32-row tiles of the swish gate's value and gate halves and of
+ *              a_to_b in turn; 7 its bias [value | gate | a_to_b]; 8 w_down [d, inner], 9 its bias
+ *   10 bias    the layer's pair bias: element b at b / bias_div * sbias, dense [heads, n, n]
+ * weights packed by bmx_x3_pack, biases fp32 or NULL.  eps (host): 2 per layer, the a_norm eps of
+ * the attention's and of the transition's AdaLN; eps_s: every s_norm's.  mask: fp32, row b at b *
+ * smask.  workspace: bmx_token_stack_workspace_bytes, 256-byte aligned. */
+size_t bmx_token_stack_workspace_bytes(int64_t batch, int64_t n, int heads, int head_dim, int64_t inner);
+int bmx_token_stack_fwd(const float* a, const float* s, int64_t batch, int64_t n, int heads, int head_dim,
+                        int64_t inner, int layers, const void* const* params, float eps_s, const float* eps,
+                        const float* mask, int64_t smask, int64_t sbias, int64_t bias_div, float inf, float* out,
+                        void* workspace, size_t workspace_bytes, bmx_stream_t stream);
+
 /* P = softmax(round(round(S + mask) + bias)) over the last axis, rounding to dtype.
  * shape = {B, I, H, Q, K}; element strides of scores [B,I,H,Q,K], bias [B,1,H,Q,K], mask [B,I,1,1,K].
  * out is contiguous.  Replaces ordered_softmax (kernels/triangle_softmax.py:117-161) and
