@@ -303,6 +303,14 @@ __device__ __forceinline__ void x3_packed_store4(bf16* op, int64_t row, int64_t 
   *(bf16x4*)(dst + 512) = lo;
 }
 
+// Packed fp32 operands (linear_f32.hip) in v_mfma_f32_32x32x2f32 order: per 32
+// rows and 8 columns one contiguous 1 KB run in which lane (row % 32) + 32 *
+// (column % 8 / 4) holds 4 columns, its values for four successive MFMAs.
+// `steps` = columns / 8.
+__host__ __device__ __forceinline__ int64_t f32_packed_index(int64_t row, int64_t col, int64_t steps) {
+  return ((row >> 5) * steps + (col >> 3)) * 256 + (((row & 31) + 32 * ((col >> 2) & 1)) << 2) + (col & 3);
+}
+
 }  // namespace bmx
 
 // ---------------------------------------------------------------------------
@@ -329,6 +337,10 @@ int gated_residual_adaln_packed(const float* a, const float* g, int64_t ldg, con
 int token_attention_packed(const float* proj, int64_t batch, int64_t n, int heads, int head_dim, const float* bias,
                            int64_t sbias, int64_t bias_div, const float* mask, int64_t smask, float inf, bf16* op,
                            void* ws, hipStream_t stream);
+// The same for the Pairformer sequence stack (fp32 kernel), the output as a
+// packed fp32 operand (f32_packed_index) of batch * n rows.
+int sequence_attention_packed(const float* proj, int64_t batch, int64_t n, int heads, int head_dim, const float* bias,
+                              const float* mask, int64_t smask, float inf, float* op, hipStream_t stream);
 size_t token_attention_workspace(int64_t batch, int64_t n, int heads, int head_dim);
 }  // namespace bmx
 

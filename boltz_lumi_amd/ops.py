@@ -1005,6 +1005,39 @@ def seq_attention_windowed(q, k, v, bias, mask, g, inf, *, windows, key_offset, 
     return out
 
 
+def f32_pack(rows, k, *parts):
+    """Packed fp32 operand of ``rows`` x ``k`` (``bmx_f32_pack``) from ``parts`` of
+    (tile0, tile stride, weight)."""
+    out = torch.empty(rows * k, device=parts[0][2].device, dtype=torch.float32)
+    for tile0, stride, w in parts:
+        w = _f32(w)
+        N.call("bmx_f32_pack", w.data_ptr(), w.shape[0], w.shape[1], w.stride(0), tile0, stride, out.data_ptr(),
+               _stream(w))
+    return out
+
+
+def sequence_stack(s, params, eps_attn, eps_trans, bias, mask, heads, hidden, inf):
+    """A PairformerLayer's fp32 sequence stack as one native call
+    (``bmx_sequence_stack_fwd``): s [B, N, d], the 9 fp32 parameter tensors
+    (None for an absent proj_q bias) in its order, bias [B, H, N, N], mask
+    [B, N]; returns the new s."""
+    _cuda(s, bias, mask, *(p for p in params if p is not None))
+    _check(s.dim() == 3 and s.dtype == torch.float32 and s.is_contiguous(), "expected contiguous fp32 s [B, N, d]")
+    b, n, d = s.shape
+    _check(len(params) == 9 and all(p is None or (p.dtype == torch.float32 and p.is_contiguous()) for p in params),
+           "expected 9 contiguous fp32 parameters")
+    _check(bias.shape == (b, heads, n, n) and bias.dtype == torch.float32 and bias.is_contiguous(),
+           "expected a contiguous fp32 [B, H, N, N] bias")
+    _check(mask.shape == (b, n) and mask.dtype == torch.float32 and mask.stride(1) == 1, "expected an fp32 [B, N] mask")
+    out = torch.empty_like(s)
+    ws = _workspace(N.lib().bmx_sequence_stack_workspace_bytes(b * n, d, hidden), s.device)
+    N.call("bmx_sequence_stack_fwd", s.data_ptr(), b, n, heads, d // heads, hidden,
+           (ctypes.c_void_p * 9)(*[0 if p is None else p.data_ptr() for p in params]), float(eps_attn),
+           float(eps_trans), bias.data_ptr(), mask.data_ptr(), mask.stride(0) if b > 1 else 0, float(inf),
+           out.data_ptr(), ws.data_ptr(), ws.numel(), _stream(s))
+    return out
+
+
 def token_stack(a, s, params, eps, eps_s, heads, inner, mask, sbias, bias_div, inf):
     """A stack of diffusion transformer layers on at most 1024 rows as one
     native call (``bmx_token_stack_fwd``): a, s [B, N, d] fp32, ``params`` the

@@ -230,6 +230,45 @@ def sequence_ok(layer, s, z, mask) -> bool:
             and mask is not None and tuple(mask.shape) == tuple(s.shape[:2]) and mask.device == z.device)
 
 
+def _layer_norm_384(norm) -> bool:
+    return (type(norm) is torch.nn.LayerNorm and _plain(norm) and "forward" not in vars(norm)
+            and tuple(norm.normalized_shape) == (384,) and norm.weight is not None and norm.bias is not None)
+
+
+def _native_sequence_params(layer, device):
+    """The 9 parameters of ``ops.sequence_stack`` where the whole sequence
+    stack (``sequence_ok`` holds) may run as that one call: plain LayerNorms,
+    an upstream Transition(384) without biases, unhooked, and fp32 contiguous
+    parameters on ``device``; else None."""
+    att, tr = layer.attention, layer.transition_s
+    if not (type(tr).__name__ == "Transition" and _plain(tr) and "forward" not in vars(tr)
+            and _layer_norm_384(layer.pre_norm_s) and _layer_norm_384(tr.norm)
+            and all(_plain(m) and "forward" not in vars(m) for m in (tr.fc1, tr.fc2, tr.fc3))
+            and _no_bias(tr.fc1, tr.fc2, tr.fc3, att.proj_k, att.proj_v, att.proj_g, att.proj_o)
+            and type(getattr(tr, "silu", None)) is torch.nn.SiLU):
+        return None
+    hidden = tr.fc1.weight.shape[0]
+    if hidden % 32 or not (_shape(tr.fc1.weight, hidden, 384) and _shape(tr.fc2.weight, hidden, 384)
+                           and _shape(tr.fc3.weight, 384, hidden)
+                           and all(_shape(m.weight, 384, 384)
+                                   for m in (att.proj_q, att.proj_k, att.proj_v, att.proj_g, att.proj_o))):
+        return None
+    sources = (att.proj_q.weight, att.proj_k.weight, att.proj_v.weight, att.proj_g.weight, att.proj_o.weight,
+               tr.fc1.weight, tr.fc2.weight, tr.fc3.weight)
+    rest = (layer.pre_norm_s.weight, layer.pre_norm_s.bias, tr.norm.weight, tr.norm.bias)
+    if not fp32_contiguous_on(device, *sources, *rest, *(() if att.proj_q.bias is None else (att.proj_q.bias,))):
+        return None
+
+    def build():
+        q, k, v, g, o, fc1, fc2, fc3 = sources
+        return (ops.f32_pack(4 * 384, 384, (0, 1, q), (12, 1, k), (24, 1, v), (36, 1, g)),
+                ops.f32_pack(384, 384, (0, 1, o)), ops.f32_pack(2 * hidden, 384, (0, 2, fc1), (1, 2, fc2)),
+                ops.f32_pack(384, hidden, (0, 1, fc3)))
+
+    qkvg, o, up, down = ops.cached_value(layer, "sequence_pack", sources, build)
+    return rest[0], rest[1], qkvg, att.proj_q.bias, o, rest[2], rest[3], up, down
+
+
 def sequence_stack(layer, s, z, mask, pair_bias=None):
     """Upstream's sequence stack in fp32 with autocast off:
     ``s + attention(pre_norm_s(s), z)``, then ``+ transition_s``, then
@@ -239,9 +278,19 @@ def sequence_stack(layer, s, z, mask, pair_bias=None):
     GEMM."""
     with torch.autocast("cuda", enabled=False):
         s = s.float()
+        seq_ok = sequence_ok(layer, s, z, mask)
+        if (seq_ok and pair_bias is not None and s.is_cuda and not torch.is_grad_enabled()
+                and not layer.training and s.shape[0] > 0 and s.shape[1] > 0):
+            params = _native_sequence_params(layer, s.device)
+            if params is not None:
+                tr, m = layer.transition_s, mask.float()
+                s = ops.sequence_stack(s.contiguous(), params, layer.pre_norm_s.eps, tr.norm.eps, pair_bias,
+                                       m if m.stride(1) == 1 else m.contiguous(), layer.attention.num_heads,
+                                       tr.fc1.weight.shape[0], layer.attention.inf)
+                return layer.s_post_norm(s)
         s_normed = layer.pre_norm_s(s)
         o = None
-        if sequence_ok(layer, s, z, mask):
+        if seq_ok:
             if pair_bias is None and pair_bias_mods(layer.attention) is not None:
                 norm, lin = pair_bias_mods(layer.attention)
                 pair_bias = torch.empty((z.shape[0], 16, z.shape[1], z.shape[2]), device=z.device,

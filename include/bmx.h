@@ -150,6 +150,27 @@ int bmx_gated_residual_adaln_split3_bf16(const float* a, const float* gate, int6
 int bmx_x3_pack(const float* w, int64_t rows, int64_t k, int64_t ldw, const float* col_scale, int64_t tile0,
                 int64_t tile_stride, void* out, bmx_stream_t stream);
 
+/* fp32 weight rows as a packed operand of the sequence stack's fp32 linears: per 32 rows and 8
+ * columns one contiguous 1 KB run in MFMA order (lane (row % 32) + 32 (column % 8 / 4) holds 4
+ * columns); 32-row tile t goes to packed tile tile0 + t * tile_stride.  rows a multiple of 32, k of
+ * 8.  No reference kernel. */
+int bmx_f32_pack(const float* w, int64_t rows, int64_t k, int64_t ldw, int64_t tile0, int64_t tile_stride, float* out,
+                 bmx_stream_t stream);
+
+/* The sequence stack of one PairformerLayer in fp32 (upstream keeps it out of autocast; the
+ * reference leaves it to torch, math as pair_bias.py:15-36): out = s1 + transition_s(s1), s1 = s +
+ * proj_o(attention(pre_norm_s(s))), for batch elements of n rows, d = heads * head_dim <= 512.
+ * params: 9 fp32 device pointers (host array): 0, 1 pre_norm_s weight, bias; 2 [proj_q; proj_k;
+ * proj_v; proj_g] [4 d, d] packed (bmx_f32_pack), 3 proj_q's bias or NULL; 4 proj_o [d, d] packed; 5, 6
+ * transition_s norm weight, bias; 7 [2 hidden, d] packed, 32-row tiles of fc1 and of fc2 in turn; 8
+ * fc3 [d, hidden] packed.  bias [batch, heads, n, n] dense (proj_z of z), mask row b at b * smask.
+ * out may not alias s; workspace: bmx_sequence_stack_workspace_bytes(batch * n, ..). */
+size_t bmx_sequence_stack_workspace_bytes(int64_t rows, int64_t d, int64_t hidden);
+int bmx_sequence_stack_fwd(const float* s, int64_t batch, int64_t n, int heads, int head_dim, int64_t hidden,
+                           const void* const* params, float eps_attn, float eps_trans, const float* bias,
+                           const float* mask, int64_t smask, float inf, float* out, void* workspace,
+                           size_t workspace_bytes, bmx_stream_t stream);
+
 /* A stack of diffusion transformer layers for few rows (batch * n <= 1024): transformersv2
  * DiffusionTransformer, whose AdaLN, attention and conditioned transition the reference patches
  * one by one (diffusion.py:52-68, pair_bias.py:15-36).  a, s, out: fp32 [batch * n, d], d =
