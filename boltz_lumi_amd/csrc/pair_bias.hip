@@ -682,6 +682,25 @@ size_t x3_workspace_bytes(int64_t batch, int64_t nk, int heads, int head_dim) {
   return 4 * ((tile + 255) / 256 * 256) + (size_t)(batch * x3_nkp(nk)) * sizeof(float);
 }
 
+// The attention proper, on K / V^T and mask terms as the pre-pass writes them.
+int launch_x3_attention(const char* name, const float* q, const bf16* kh, const bf16* kl, const bf16* vth,
+                        const bf16* vtl, const float* mterm, const float* bias, const float* g, int64_t batch,
+                        const SeqAttnShape& sh, int heads, int head_dim, float* out, bf16* op, bool packed,
+                        hipStream_t stream) {
+  const bool vec = (uintptr_t)bias % 4 == 0;  // 16-byte bias loads, at any row alignment
+  const int64_t items = (batch + sh.bdiv - 1) / sh.bdiv * sh.bdiv * heads * ((sh.nq + kX3Q - 1) / kX3Q);
+  const dim3 grid((unsigned)(8 * ((items + 7) / 8)));
+  const float rscale = 1.f / sqrtf((float)head_dim);
+#define SEQ_ATTN_X3(DIM)                                                                                       \
+  seq_attention_x3_kernel<DIM><<<grid, 256, 0, stream>>>(q, kh, kl, vth, vtl, mterm, bias, g, sh, heads, batch, \
+                                                         rscale, vec, out, op, packed)
+  if (head_dim == 24) SEQ_ATTN_X3(24);
+  else if (head_dim == 32) SEQ_ATTN_X3(32);
+  else SEQ_ATTN_X3(48);
+#undef SEQ_ATTN_X3
+  return check_launch(name);
+}
+
 int launch_seq_attention_x3(const char* name, const float* q, const float* k, const float* v, const float* bias,
                             const float* mask, const float* g, int64_t batch, const SeqAttnShape& sh, int heads,
                             int head_dim, float inf, float* out, bf16* op, void* ws, hipStream_t stream,
@@ -706,18 +725,8 @@ int launch_seq_attention_x3(const char* name, const float* q, const float* k, co
   else SEQ_ATTN_SPLIT(false, 1);
 #undef SEQ_ATTN_SPLIT
   if (int rc = check_launch(name)) return rc;
-  const bool vec = (uintptr_t)bias % 4 == 0;  // 16-byte bias loads, at any row alignment
-  const int64_t items = (batch + sh.bdiv - 1) / sh.bdiv * sh.bdiv * heads * ((sh.nq + kX3Q - 1) / kX3Q);
-  const dim3 grid((unsigned)(8 * ((items + 7) / 8)));
-  const float rscale = 1.f / sqrtf((float)head_dim);
-#define SEQ_ATTN_X3(DIM)                                                                                       \
-  seq_attention_x3_kernel<DIM><<<grid, 256, 0, stream>>>(q, kh, kl, vth, vtl, mterm, bias, g, sh, heads, batch, \
-                                                         rscale, vec, out, op, packed)
-  if (head_dim == 24) SEQ_ATTN_X3(24);
-  else if (head_dim == 32) SEQ_ATTN_X3(32);
-  else SEQ_ATTN_X3(48);
-#undef SEQ_ATTN_X3
-  return check_launch(name);
+  return launch_x3_attention(name, q, kh, kl, vth, vtl, mterm, bias, g, batch, sh, heads, head_dim, out, op, packed,
+                             stream);
 }
 
 // From this many keys on the split-bf16 kernel runs the token attention (as
@@ -728,6 +737,15 @@ constexpr int64_t kX3MinKeys = 256;
 }  // namespace
 
 namespace bmx {
+
+int seq_attention_x3_presplit(const char* name, const float* q, const float* g, int64_t ldq, int64_t sq, int64_t batch,
+                              int64_t n, int heads, int head_dim, const float* bias, int64_t bias_div, const bf16* kh,
+                              const bf16* kl, const bf16* vth, const bf16* vtl, const float* mterm, float* out,
+                              hipStream_t stream) {
+  const SeqAttnShape sh{(int)n, (int)n, (int)bias_div, ldq, 0, sq, 0, heads * n * n, 0};
+  return launch_x3_attention(name, q, kh, kl, vth, vtl, mterm, bias, g, batch, sh, heads, head_dim, out, nullptr, false,
+                             stream);
+}
 
 size_t token_attention_workspace(int64_t batch, int64_t n, int heads, int head_dim) {
   return n >= kX3MinKeys ? x3_workspace_bytes(batch, n, heads, head_dim) : 0;

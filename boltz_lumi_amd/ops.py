@@ -657,31 +657,40 @@ def triattn(module, x, mask, starting, out_mode=OUT_BF16, out=None, workspace=No
     return out
 
 
-TRIATTN_FP32_PROJ_COLS = 576
+def _triattn_fp32_split_weights(module):
+    """fp32 mode's projections for ``bmx_triattn_fp32_fwd``: q | k | v | g packed
+    as a split operand, their biases and the triangle bias's [512 + 4], and the
+    triangle-bias rows as bf16 [high, low][16][128]."""
+    mha = module.mha
+    lins = (mha.linear_q, mha.linear_k, mha.linear_v, mha.linear_g)
 
-
-def _triattn_fp32_split_weight(module):
-    """q | k | v | g and the triangle bias as one split-bf16 weight for
-    LayerNorm-without-affine(x), the LayerNorm affine folded in:
-    (W diag w) LN0(x) + (bias + W b); bf16 [576, 3 * 128 + 64] (rows 512 ..
-    512 + heads the triangle bias, zero rows up to 576)."""
-    mha, ln = module.mha, module.layer_norm
-    lins = (mha.linear_q, mha.linear_k, mha.linear_v, mha.linear_g, module.linear)
-
-    def fold(*_):
-        w = torch.cat([lin.weight.detach().float() for lin in lins])
+    def build():
+        w = torch.empty(2 * 4 * C * C, device=mha.linear_q.weight.device, dtype=torch.bfloat16)
+        for i, lin in enumerate(lins):
+            x3_pack(w, i * C // 32, lin.weight)
         b = torch.cat([lin.bias.detach().float() if lin.bias is not None
-                       else w.new_zeros(lin.out_features) for lin in lins])
-        if ln.bias is not None:
-            b = b + w @ ln.bias.detach().float()
-        # zero rows up to 576 outputs: the GEMM runs faster than at 516 and output rows stay 128-byte aligned
-        pad = TRIATTN_FP32_PROJ_COLS - w.shape[0]
-        w = torch.cat([w * ln.weight.detach().float(), w.new_zeros(pad, C)])
-        return _x3_weight(w, torch.cat([b, b.new_zeros(pad)]))
+                       else lin.weight.new_zeros(lin.out_features, dtype=torch.float32)
+                       for lin in lins + (module.linear,)])
+        rows = module.linear.weight.detach().float()
+        rows = torch.cat([rows, rows.new_zeros(16 - rows.shape[0], C)])
+        hi = rows.to(torch.bfloat16)
+        return w, b, torch.stack([hi, (rows - hi.float()).to(torch.bfloat16)]).contiguous()
 
-    srcs = tuple(t for m_ in (ln,) + lins for t in (m_.weight, m_.bias) if t is not None)
-    _check(4 * C + module.no_heads <= TRIATTN_FP32_PROJ_COLS, "too many heads")
-    return cached_weight(module, "qkvgb_ln_x3", srcs, fold)
+    srcs = tuple(t for lin in lins + (module.linear,) for t in (lin.weight, lin.bias) if t is not None)
+    return cached_value(module, "fp32_proj_x3", srcs, build)
+
+
+def _triattn_fp32_native(module, x, mask, starting, tri_bias, stages, row0, rows, out=None, ws=None):
+    """One ``bmx_triattn_fp32_fwd`` call on frame rows row0 .. row0 + rows - 1."""
+    w, b, wb = _triattn_fp32_split_weights(module)
+    ln = module.layer_norm
+    lnw = _f32(ln.weight)
+    lnb = None if ln.bias is None else _f32(ln.bias)
+    N.call("bmx_triattn_fp32_fwd", x.data_ptr(), None if mask is None else mask.data_ptr(), x.shape[0], int(starting),
+           row0, rows, float(module.inf), lnw.data_ptr(), None if lnb is None else lnb.data_ptr(), float(ln.eps),
+           w.data_ptr(), b.data_ptr(), wb.data_ptr(), tri_bias.data_ptr(), stages,
+           None if out is None else out.data_ptr(), None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+           _stream(x))
 
 
 def _triattn_fp32_exact_weights(module):
@@ -697,16 +706,16 @@ def _triattn_fp32_exact_weights(module):
 def triattn_fp32(module, x, mask, starting, block_rows=None):
     """TriangleAttention (starting or ending node) in fp32 for x [N, N, 128]
     fp32, the fp32 mode of the module (autocast off; reference
-    triangle.py:38-52 accelerates it too).  The q | k | v | g projection and
-    the triangle bias are one split-bf16 GEMM of LayerNorm-without-affine(x),
-    the LayerNorm affine folded into its weights (in exact fp32 mode the fp32
-    LN128 kernel and fp32 GEMMs);
-    the attention, mask bias, softmax, PV product and gate run fused in
-    ``bmx_seq_attention_x3_batched_fwd`` (split-bf16 products, about 2^-16
-    relative each; ``bmx_seq_attention_batched_fwd`` on fp32 MFMA in exact fp32
-    mode), every row i one batch element attending over its N keys, all rows
-    sharing the [4, N, N] triangle bias, so the [N, 4, N, N] scores never
-    reach HBM; ``linear_o`` is an fp32 GEMM.  Returns fp32 [N, N, 128].
+    triangle.py:38-52 accelerates it too).  One kernel normalises x, projects
+    q | k | v | g and the triangle bias with split-bf16 products (about 2^-16
+    relative each) and writes the attention's operands
+    (``bmx_triattn_fp32_fwd``; the ending node reads x's columns in place); the
+    attention, mask bias, softmax, PV product and gate run fused on the
+    split-bf16 kernel, every row i one batch element attending over its N keys,
+    all rows sharing the [4, N, N] triangle bias, so the [N, 4, N, N] scores
+    never reach HBM; ``linear_o`` is an fp32 GEMM.  In exact fp32 mode the fp32
+    LN128 kernel, fp32 GEMMs and the fp32-MFMA attention run instead.  Returns
+    fp32 [N, N, 128].
 
     ``block_rows`` < N processes the rows of the frame (x's rows for the
     starting node, its columns for the ending node) in blocks of that many
@@ -720,80 +729,89 @@ def triattn_fp32(module, x, mask, starting, block_rows=None):
     _check(heads * d == C, "expected heads x head dim = 128")
     if block_rows is not None and 0 < block_rows < n:
         return _triattn_fp32_blocked(module, x, mask, starting, int(block_rows))
+    ln = module.layer_norm
+    if not _EXACT_FP32[0] and ln.weight is not None and heads == 4:
+        return _triattn_fp32_split(module, x.contiguous(), mask, starting, n)
     if not starting:
         mask = None if mask is None else mask.transpose(0, 1)
-    ln = module.layer_norm
-    split = not _EXACT_FP32[0] and ln.weight is not None
-    # the ending node works on x transposed: the split path's LayerNorm reads the transposed rows in
-    # place, the exact path transposes x once
-    x = x.contiguous() if starting or split else x.transpose(0, 1).contiguous()
-    if split:
-        w3 = _triattn_fp32_split_weight(module)
-        op = (layernorm_split3(x.view(-1, C), ln.eps) if starting
-              else layernorm_split3_t(x, ln.eps).view(-1, split_width(C)))
-        proj = mm_split(op, w3).view(n, n, TRIATTN_FP32_PROJ_COLS)
-        del op  # 0.9 KB per pair, not needed by the attention
-        tri_bias = proj[..., 4 * C:4 * C + heads].permute(2, 0, 1).contiguous()  # [H, q, k], shared by every row
-    else:
-        xn = norm(x.view(-1, C), _f32(ln.weight), _f32(ln.bias), ln.eps, bf16_output=False)
-        w, b = _triattn_fp32_exact_weights(module)
-        proj = torch.nn.functional.linear(xn, w, b).view(n, n, 4 * C)
-        tri_bias = torch.nn.functional.linear(xn, module.linear.weight.float()).view(n, n, heads)
-        tri_bias = tri_bias.permute(2, 0, 1).contiguous()  # [H, q, k], shared by every row
+        x = x.transpose(0, 1)
+    x = x.contiguous()
+    xn = norm(x.view(-1, C), _f32(ln.weight), _f32(ln.bias), ln.eps, bf16_output=False)
+    w, b = _triattn_fp32_exact_weights(module)
+    proj = torch.nn.functional.linear(xn, w, b).view(n, n, 4 * C)
+    tri_bias = torch.nn.functional.linear(xn, module.linear.weight.float()).view(n, n, heads)
+    tri_bias = tri_bias.permute(2, 0, 1).contiguous()  # [H, q, k], shared by every row
     m = x.new_ones(n, n) if mask is None else mask.to(torch.float32).contiguous()
-    q, k, v, g = proj[..., :4 * C].split(C, dim=-1)
-    # the split-bf16 kernel (about 2^-16 relative per product; 1.8x faster at N = 1024) unless exact
-    # fp32 products are asked for
+    q, k, v, g = proj.split(C, dim=-1)
     o = seq_attention_batched(q, k, v, tri_bias[None], m, g, module.inf, bias_div=n, split=not _EXACT_FP32[0])
     del q, k, v, g, proj, tri_bias  # 2.3 KB per pair, before linear_o's output is allocated
     out = torch.nn.functional.linear(o, mha.linear_o.weight.float(), mha.linear_o.bias.float())
     return out if starting else out.transpose(0, 1)
 
 
+def _triattn_fp32_split(module, x, mask, starting, rows):
+    """``triattn_fp32`` on split-bf16 products in blocks of ``rows`` frame rows
+    (all of them in one block: one kernel writes the triangle bias, which every
+    row shares, beside the rows' operands; several blocks: a first pass writes
+    it for all rows)."""
+    n, mha = x.shape[0], module.mha
+    m = None if mask is None else mask.to(torch.float32).contiguous()
+    tri_bias = torch.empty(4, n, n, device=x.device, dtype=torch.float32)
+    ws = _workspace(N.lib().bmx_triattn_fp32_workspace_bytes(n, rows), x.device)
+    w_o, b_o = mha.linear_o.weight.float(), mha.linear_o.bias.float()
+    if rows >= n:
+        o = torch.empty(n, n, C, device=x.device, dtype=torch.float32)
+        if n:
+            _triattn_fp32_native(module, x, m, starting, tri_bias, 3, 0, n, o, ws)
+        del ws, tri_bias  # 2 KB per pair, before linear_o's output is allocated
+        out = torch.nn.functional.linear(o, w_o, b_o)
+    else:
+        _triattn_fp32_native(module, x, m, starting, tri_bias, 1, 0, n)
+        o = torch.empty(rows, n, C, device=x.device, dtype=torch.float32)
+        out = torch.empty(n, n, C, device=x.device, dtype=torch.float32)  # the output frame
+        for i0 in range(0, n, rows):
+            r = min(rows, n - i0)
+            _triattn_fp32_native(module, x, m, starting, tri_bias, 2, i0, r, o, ws)
+            torch.addmm(b_o, o[:r].view(-1, C), w_o.t(), out=out[i0:i0 + r].view(-1, C))
+    return out if starting else out.transpose(0, 1)
+
+
 def _triattn_fp32_blocked(module, x, mask, starting, rows):
     """``triattn_fp32`` over blocks of ``rows`` frame rows (x's rows for the
-    starting node, x's columns, copied transposed one block at a time, for the
-    ending node).  A first pass writes the [H, N, N] triangle bias, which every
-    row shares, from each block's LayerNorm operand and only the bias rows of
-    the projection weight; a second pass recomputes each block's operand and
-    runs its q | k | v | g projection, the fused attention over the block's
-    rows and ``linear_o`` into the output frame.  Full-frame memory: the
-    output, the bias and the mask (about 532 bytes per pair); the rest is
-    per block."""
+    starting node, x's columns for the ending node).  A first pass writes the
+    [H, N, N] triangle bias, which every row shares; a second pass runs each
+    block's projection, the fused attention over the block's rows and
+    ``linear_o`` into the output frame.  Full-frame memory: the output, the
+    bias and the mask (about 532 bytes per pair); the rest is per block.  Exact
+    fp32 mode copies the ending node's columns transposed one block at a time
+    and computes the bias from each block's LayerNorm and only the bias rows of
+    the projection weight."""
     n = x.size(0)
     mha, heads, ln = module.mha, module.no_heads, module.layer_norm
-    split = not _EXACT_FP32[0] and ln.weight is not None
+    if not _EXACT_FP32[0] and ln.weight is not None and heads == 4:
+        return _triattn_fp32_split(module, x.contiguous(), mask, starting, rows)
     if mask is None:
         m = x.new_ones(n, n)
     else:
         m = (mask if starting else mask.transpose(0, 1)).to(torch.float32).contiguous()
 
-    def frame_rows(i0, i1):  # [i1 - i0, N, 128] fp32, contiguous
-        return x[i0:i1].contiguous() if starting else x[:, i0:i1].transpose(0, 1).contiguous()
+    def features(i0, i1):  # LayerNorm of frame rows i0 .. i1 - 1: [(i1 - i0) N, 128] fp32
+        xb = x[i0:i1].contiguous() if starting else x[:, i0:i1].transpose(0, 1).contiguous()
+        return norm(xb.view(-1, C), _f32(ln.weight), _f32(ln.bias), ln.eps, bf16_output=False)
 
-    if split:
-        w3 = _triattn_fp32_split_weight(module)
-        w3_bias = w3[4 * C:]  # the bias rows and their zero padding: 64 outputs
-        features = lambda xb: layernorm_split3(xb.view(-1, C), ln.eps)
-        project_bias = lambda f: mm_split(f, w3_bias)
-        project = lambda f: mm_split(f, w3)
-    else:
-        w, b = _triattn_fp32_exact_weights(module)
-        w_bias = module.linear.weight.float()
-        features = lambda xb: norm(xb.view(-1, C), _f32(ln.weight), _f32(ln.bias), ln.eps, bf16_output=False)
-        project_bias = lambda f: torch.nn.functional.linear(f, w_bias)
-        project = lambda f: torch.nn.functional.linear(f, w, b)
+    w, b = _triattn_fp32_exact_weights(module)
+    w_bias = module.linear.weight.float()
     blocks = [(i0, min(n, i0 + rows)) for i0 in range(0, n, rows)]
     tri_bias = torch.empty(heads, n, n, device=x.device, dtype=torch.float32)  # [H, q, k]
     for i0, i1 in blocks:
-        bias = project_bias(features(frame_rows(i0, i1)))[:, :heads]
+        bias = torch.nn.functional.linear(features(i0, i1), w_bias)
         tri_bias[:, i0:i1] = bias.view(i1 - i0, n, heads).permute(2, 0, 1)
         del bias
     out = torch.empty(n, n, C, device=x.device, dtype=torch.float32)  # the output frame
     w_o, b_o = mha.linear_o.weight.float(), mha.linear_o.bias.float()
     for i0, i1 in blocks:
-        proj = project(features(frame_rows(i0, i1))).view(i1 - i0, n, -1)
-        q, k, v, g = proj[..., :4 * C].split(C, dim=-1)
+        proj = torch.nn.functional.linear(features(i0, i1), w, b).view(i1 - i0, n, -1)
+        q, k, v, g = proj.split(C, dim=-1)
         o = seq_attention_batched(q, k, v, tri_bias[None], m[i0:i1], g, module.inf, bias_div=i1 - i0,
                                   split=not _EXACT_FP32[0])
         del q, k, v, g, proj

@@ -30,10 +30,11 @@ def _native_shape_ok(module, x) -> bool:
 
 
 # fp32 mode holds at most this many bytes per pair at its peak (``ops.triattn_fp32``:
-# the [N^2, 576] fp32 projection, the split-bf16 attention's K / V workspace,
-# the attention output and the linear_o result), all N rows at once.  Measured
-# at N = 1024: 3860-3864 bytes per pair by default, 3088-3604 with exact fp32
-# linears (tests/test_gpu_fp32_triattn.py); the bound keeps a margin.
+# q, g and the split K / V, the triangle bias, the attention output and the
+# linear_o result; in exact fp32 mode the [N^2, 512] projection beside them), all
+# N rows at once.  Measured at N = 1024: 2584 bytes per pair by default,
+# 3088-3604 with exact fp32 linears (tests/test_gpu_fp32_triattn.py); the bound
+# keeps a margin.
 FP32_BYTES_PER_PAIR = 4608
 # ... and runs in one pass while that fits in this share of the device memory
 # (N up to about 5500 on a 288 GiB MI355X).  Larger N run in blocks of frame
@@ -65,10 +66,8 @@ def triangle_attention_forward(self, x, mask=None, chunk_size=None, use_kernels=
     Native in inference under bf16 autocast (or for bf16 x), with a bf16
     result like the upstream autocast path; and in fp32 mode (autocast off,
     fp32 x; reference triangle.py:38-52), with an fp32 result
-    (``ops.triattn_fp32``): by default one split-bf16 GEMM of
-    LayerNorm-without-affine(x) for q | k | v | g and the triangle bias (the
-    LayerNorm affine folded into the weights) and the fused split-bf16
-    attention, about 2^-16 relative per product; with
+    (``ops.triattn_fp32``): by default one kernel from x to the operands of the
+    fused split-bf16 attention, about 2^-16 relative per product; with
     ``BMX_EXACT_FP32_LINEARS=1`` the fp32 LN128 kernel, fp32 GEMMs and the
     fp32-MFMA attention.  fp32 mode runs all N rows in one pass while that
     working set fits (``fp32_native_fits``) and in blocks of rows above

@@ -150,6 +150,20 @@ int bmx_gated_residual_adaln_split3_bf16(const float* a, const float* gate, int6
 int bmx_x3_pack(const float* w, int64_t rows, int64_t k, int64_t ldw, const float* col_scale, int64_t tile0,
                 int64_t tile_stride, void* out, bmx_stream_t stream);
 
+/* fp32-mode triangle attention (TriangleAttention with autocast off; reference
+ * triangle.py:38-52) up to linear_o: LayerNorm, the q | k | v | g and triangle-bias projections and
+ * the attention with its gate, products in split bf16 (about 2^-16 relative), for the frame rows
+ * row0 .. row0 + rows - 1 of x [n, n, 128] (x's rows for the starting node, its columns for the
+ * ending node).  w_qkvg: the four 128 x 128 weights packed by bmx_x3_pack (512 x 128), b_qkvg fp32
+ * [512 + 4], the last 4 the triangle bias's; w_bias: the triangle-bias rows as bf16 [high, low][16][128] (rows past 4 zero).  stages:
+ * 1 writes the rows' triangle bias into tri_bias [4, n, n], 2 attends (tri_bias complete) into out
+ * [rows, n, 128], 3 both (all rows).  workspace (stage 2): bmx_triattn_fp32_workspace_bytes. */
+size_t bmx_triattn_fp32_workspace_bytes(int64_t n, int64_t rows);
+int bmx_triattn_fp32_fwd(const float* x, const float* mask, int64_t n, int starting, int64_t row0, int64_t rows,
+                         float inf, const float* ln_w, const float* ln_b, float eps, const void* w_qkvg,
+                         const float* b_qkvg, const void* w_bias, float* tri_bias, int stages, float* out,
+                         void* workspace, size_t workspace_bytes, bmx_stream_t stream);
+
 /* fp32 weight rows as a packed operand of the sequence stack's fp32 linears: per 32 rows and 8
  * columns one contiguous 1 KB run in MFMA order (lane (row % 32) + 32 (column % 8 / 4) holds 4
  * columns); 32-row tile t goes to packed tile tile0 + t * tile_stride.  rows a multiple of 32, k of

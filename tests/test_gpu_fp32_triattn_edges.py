@@ -1,0 +1,38 @@
+"""fp32-mode triangle attention's projection kernel at the edges of its 64-pair
+tiles, in blocks of rows, with and without a mask, against the oracle module
+in fp32 on the GPU."""
+
+import pytest
+import torch
+
+from boltz_lumi_amd import ops
+from oracle import boltz_ref as R
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 2, 31, 63, 64, 65, 129, 200])
+@pytest.mark.parametrize("starting", [True, False])
+@pytest.mark.parametrize("masked", [None, "tokens", "random"])
+def test_fp32_projection_edges(gpu, n, starting, masked):
+    g = torch.Generator().manual_seed(n + 3 * starting)
+    cls = R.TriangleAttention if starting else R.TriangleAttentionEndingNode
+    layer = R.randomize(cls(128, 32, 4), generator=g).to(gpu).eval()
+    x = torch.randn(n, n, 128, generator=g).to(gpu)
+    mask = None
+    if masked == "tokens":  # padded tokens: closed rows too
+        tok = torch.ones(n)
+        tok[n - n // 5:] = 0
+        mask = (tok[:, None] * tok[None, :]).to(gpu)
+    elif masked == "random":
+        mask = (torch.rand(n, n, generator=g) > 0.3).float().to(gpu)
+    with torch.inference_mode():
+        got = ops.triattn_fp32(layer, x, mask, starting)
+        blocked = ops.triattn_fp32(layer, x, mask, starting, block_rows=max(1, n // 3))
+        want = layer(x[None], None if mask is None else mask[None])[0]
+    assert torch.isfinite(got).all()
+    # the same products row by row; linear_o's library GEMM sums its 128 fp32 products in an order that depends on
+    # its shape (2^-24 each)
+    assert (got - blocked).abs().max() / got.abs().max() < 1e-6
+    err = ((got - want).abs().max() / want.abs().max()).item()
+    assert err < 1e-4, err  # split products: 2^-16 relative each
