@@ -411,54 +411,97 @@ def _stack_pack(layer, d, inner):
             pack(d, inner, (0, 1, down.weight, None)), biases([(down, down.bias)]))
 
 
-def _stack_sources(layer):
-    att, tr = layer.pair_bias_attn, layer.transition
-    lins = (att.proj_q, att.proj_k, att.proj_v, att.proj_g, att.proj_o, tr.swish_gate[0], tr.a_to_b,
-            tr.b_to_a) + _gate_linears(layer)
-    return _mods_sources(layer) + tuple(p for lin in lins for p in (lin.weight, lin.bias) if p is not None)
+def _params(*modules):
+    return [p for m in modules for p in (m._parameters.get("weight"), m._parameters.get("bias")) if p is not None]
 
 
-def _native_stack(layers, a, s, biases, mask, multiplicity):
-    """The whole stack as one ``bmx_token_stack_fwd`` call, or None where it
-    does not apply: layers whose chain already runs on split operands
-    (``_with_side_ok``, ``_operand_path``) with plain proj_o and Identity
-    post_lnorm, one shape, one s_norm eps and one attention inf throughout, and
-    at most ``TOKEN_STACK_MAX_ROWS`` rows.  ``biases``: every layer's pair bias
-    as its attention's proj_z takes it."""
-    b, n, d = a.shape
-    first = layers[0].pair_bias_attn
-    heads, inner = first.num_heads, layers[0].transition.a_to_b.out_features
-    eps_s, inf = layers[0].adaln.s_norm.eps, first.inf
-    if d % 32 or inner % 32 or first.c_s != d:
+def _adaln_parts(adaln, c):
+    """(s_norm, s_scale, s_bias, eps of a_norm) of an AdaLN that
+    ``_adaln_foldable`` accepts, else None; children read from ``_modules``
+    (nn.Module.__getattr__ costs more than the checks)."""
+    kids = adaln._modules
+    an, sn, scale, shift = kids.get("a_norm"), kids.get("s_norm"), kids.get("s_scale"), kids.get("s_bias")
+    fwd = adaln.__dict__.get("forward")
+    if (not _plain(adaln) or (fwd is not None and getattr(fwd, "__func__", None) is not adaln_forward)
+            or not isinstance(an, torch.nn.LayerNorm) or an._parameters.get("weight") is not None
+            or an._parameters.get("bias") is not None
+            or not isinstance(sn, torch.nn.LayerNorm) or tuple(sn.normalized_shape) != (c,)
+            or not (_untouched(sn) and _untouched(scale) and _untouched(shift))):
         return None
+    return sn, scale, shift, an.eps
+
+
+def _stack_layer(layer, d):
+    """What ``bmx_token_stack_fwd`` needs of one layer: (attention, eps of the
+    two a_norms, eps of s_norm, inner width, source parameters of its pack), or
+    None where the layer does not run on the operand path (the conditions of
+    ``_with_side_ok`` and ``_operand_path``) with a plain proj_o and an Identity
+    post_lnorm."""
+    kids = layer._modules
+    att, tr, post, gate = (kids.get("pair_bias_attn"), kids.get("transition"), kids.get("post_lnorm"),
+                           kids.get("output_projection_linear"))
+    if (layer.training or type(post) is not torch.nn.Identity or not _untouched(post) or not operand_ok(att)
+            or not _untouched(gate) or not _plain(kids["output_projection"]) or tr.training
+            or not _patched_with(tr, transition_forward) or not _plain(tr)):
+        return None
+    tkids = tr._modules
+    oproj, swish = tkids["output_projection"], tkids["swish_gate"]
+    gate_t, sw, up, down = oproj._modules["0"], swish._modules["0"], tkids["a_to_b"], tkids["b_to_a"]
+    first, second = _adaln_parts(kids["adaln"], d), _adaln_parts(tkids["adaln"], d)
+    if first is None or second is None or not _plain(oproj) or not _untouched(gate_t) or first[0].eps != second[0].eps:
+        return None
+    akids = att._modules
+    proj_o = akids["proj_o"]
+    inner = up.out_features
+    if (not _untouched(proj_o) or inner % 32 or tuple(sw._parameters["weight"].shape) != (2 * inner, d)
+            or tuple(down._parameters["weight"].shape) != (d, inner)):
+        return None
+    sources = _params(*first[:3], *second[:3], gate, gate_t, akids["proj_q"], akids["proj_k"], akids["proj_v"],
+                      akids["proj_g"], proj_o, sw, up, down)
+    return att, first[3], second[3], first[0].eps, inner, sources
+
+
+def _native_stack(layers, a, s, bias, mask, multiplicity):
+    """The whole stack as one ``bmx_token_stack_fwd`` call, or None where it
+    does not apply: every layer as ``_stack_layer`` accepts it, one shape, one
+    s_norm eps and one attention inf throughout, linears that run split
+    (``ops.use_split``), a prepacked pair bias (dense per layer) and at most
+    ``TOKEN_STACK_MAX_ROWS`` rows.  ``bias``: [B, N, N, layers, heads]."""
+    b, n, d = a.shape
+    if d % 32 or a.shape != s.shape or not ops.use_split(d) or not 0 < b * n <= TOKEN_STACK_MAX_ROWS or mask is None:
+        return None
+    parts = []
     for layer in layers:
-        att, tr = layer.pair_bias_attn, layer.transition
-        if not (type(layer.post_lnorm) is torch.nn.Identity and _untouched(layer.post_lnorm) and _untouched(att.proj_o)
-                and att.num_heads == heads and att.c_s == d and att.inf == inf and layer.adaln.s_norm.eps == eps_s
-                and tr.a_to_b.out_features == inner and tuple(tr.swish_gate[0].weight.shape) == (2 * inner, d)
-                and tuple(tr.b_to_a.weight.shape) == (d, inner)):
+        part = _stack_layer(layer, d)
+        if part is None:
             return None
+        parts.append(part)
+    att, _, _, eps_s, inner, _ = parts[0]
+    heads, inf = att.num_heads, att.inf
     m = mask.float()
     if m.dim() != 2 or m.shape[1] != n or m.shape[0] not in (1, b):
         return None
     if m.stride(1) != 1:
         m = m.contiguous()
-    params, keep, eps, sbias = [], [m], [], None
-    for layer, z in zip(layers, biases):
-        att = layer.pair_bias_attn
-        zb = att.proj_z(z)
+    addresses, keep, eps, sbias = [], [], [], None
+    for i, (att, eps_a, eps_t, es, inn, sources) in enumerate(parts):
+        if att.num_heads != heads or att.c_s != d or att.inf != inf or es != eps_s or inn != inner:
+            return None
+        zb = att._modules["proj_z"](bias[:, :, :, i])
         if not (zb.dtype == torch.float32 and zb.dim() == 4 and zb.shape[0] * multiplicity == b
-                and tuple(zb.shape[1:]) == (heads, n, n) and zb.device == a.device and zb[0].is_contiguous()):
+                and zb.shape[1:] == (heads, n, n) and zb.device == a.device
+                and (zb.stride()[1:] == (n * n, n, 1) or zb[0].is_contiguous())):
             return None
         stride = zb.stride(0) if zb.shape[0] > 1 else 0
         if sbias is not None and stride != sbias:
             return None
         sbias = stride
-        pack = ops.cached_value(layer, "token_stack", _stack_sources(layer), lambda: _stack_pack(layer, d, inner))
+        pack = ops.cached_value(layers[i], "token_stack", sources, lambda: _stack_pack(layers[i], d, inner))
         keep += [zb, pack]
-        params += [0 if t is None else t.data_ptr() for t in pack] + [zb.data_ptr()]
-        eps += [layer.adaln.a_norm.eps, layer.transition.adaln.a_norm.eps]
-    return ops.token_stack(a, s, params, eps, eps_s, heads, inner, m, sbias, multiplicity, inf)
+        addresses += [0 if t is None else t.data_ptr() for t in pack]
+        addresses.append(zb.data_ptr())
+        eps += [eps_a, eps_t]
+    return ops.token_stack(a, s, addresses, eps, eps_s, heads, inner, m, sbias, multiplicity, inf)
 
 
 def stack_forward(self, a, s, bias=None, mask=None, to_keys=None, multiplicity=1):
@@ -473,15 +516,14 @@ def stack_forward(self, a, s, bias=None, mask=None, to_keys=None, multiplicity=1
     if getattr(self, "pair_bias_attn", True):
         n_b, n, m, d = bias.shape
         bias = bias.view(n_b, n, m, len(layers), d // len(layers))
+    if to_keys is None and a.dim() == 3 and getattr(self, "pair_bias_attn", True):
+        out = _native_stack(layers, a, s, bias, mask, multiplicity)
+        if out is not None:
+            return out
     side = _Side(s)
     # consecutive layers on the operand path chain their boundary passes: layer
     # i's last residual update also writes layer i + 1's attention operand
     chain = [_with_side_ok(l, a, s) and _operand_path(l, side, to_keys) for l in layers]
-    if (all(chain) and mask is not None and a.dim() == 3 and 0 < a.shape[0] * a.shape[1] <= TOKEN_STACK_MAX_ROWS
-            and getattr(self, "pair_bias_attn", True)):
-        out = _native_stack(layers, a, s, [bias[:, :, :, i] for i in range(len(layers))], mask, multiplicity)
-        if out is not None:
-            return out
     carry = None
     for i, layer in enumerate(layers):
         bias_l = bias[:, :, :, i] if getattr(self, "pair_bias_attn", True) else None

@@ -29,8 +29,16 @@ C = 128
 # ---------------------------------------------------------------- helpers
 
 
+# The current stream's handle by device index: what
+# ``torch.cuda.current_stream(device).cuda_stream`` returns, without building a
+# Stream object per call (2 us of a 20-us call).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
 
 
 def _code(dtype: torch.dtype) -> int:
@@ -47,10 +55,12 @@ def _check(cond: bool, msg: str) -> None:
 
 
 def _cuda(*tensors: torch.Tensor) -> None:
-    dev = tensors[0].device
+    dev = tensors[0].get_device()
     for t in tensors:
-        _check(t.is_cuda, "expected CUDA (HIP) tensors")
-        _check(t.device == dev, "all tensors must be on the same device")
+        if not t.is_cuda:
+            raise RuntimeError("expected CUDA (HIP) tensors")
+        if t.get_device() != dev:
+            raise RuntimeError("all tensors must be on the same device")
 
 
 def _inference_only() -> None:
@@ -58,12 +68,24 @@ def _inference_only() -> None:
 
 
 def cached_value(module, name: str, sources, build):
-    """``build()`` cached on ``module`` under ``name`` by the rule of
-    ``cached_weight`` (any value, e.g. several packed weights at once)."""
-    if any(p.is_inference() for p in sources):
+    """``build()``: derived weights (e.g. a bf16 concatenation, or several packed
+    weights at once), cached on ``module`` under ``name``.
+
+    Reused only while every source parameter keeps its identity, version
+    counter, storage and dtype (the rule of the reference's joint projection
+    cache, multiplication.py:29-40, plus the storage address, which a
+    ``param.data = ...`` swap changes; an address belongs to one device).
+    Inference tensors (parameters made or loaded under
+    ``torch.inference_mode``) carry no version counter, so an in-place update of
+    one cannot be seen: with such a source the value is rebuilt on every call
+    and never cached."""
+    try:
+        key = [(id(p), p._version, p.data_ptr(), p.dtype) for p in sources]
+    except RuntimeError:  # no version counter
+        if not any(p.is_inference() for p in sources):
+            raise
         with torch.no_grad():
             return build()
-    key = tuple((id(p), p._version, p.data_ptr(), p.device, p.dtype) for p in sources)
     cache = module.__dict__.setdefault("_bmx_weight_cache", {})
     hit = cache.get(name)
     if hit is None or hit[0] != key:
@@ -75,27 +97,8 @@ def cached_value(module, name: str, sources, build):
 
 
 def cached_weight(module, name: str, sources, build):
-    """Derived weight (e.g. a bf16 concatenation) cached on ``module``.
-
-    Reused only while every source parameter keeps its identity, version
-    counter, storage, device and dtype (the rule of the reference's joint
-    projection cache, multiplication.py:29-40, plus the storage address, which
-    a ``param.data = ...`` swap changes).  Inference tensors (parameters made
-    or loaded under ``torch.inference_mode``) carry no version counter, so an
-    in-place update of one cannot be seen: with such a source the weight is
-    rebuilt on every call and never cached."""
-    if any(p.is_inference() for p in sources):
-        with torch.no_grad():
-            return build(*sources).contiguous()
-    key = tuple((id(p), p._version, p.data_ptr(), p.device, p.dtype) for p in sources)
-    cache = module.__dict__.setdefault("_bmx_weight_cache", {})
-    hit = cache.get(name)
-    if hit is None or hit[0] != key:
-        with torch.no_grad():
-            value = build(*sources).contiguous()
-        hit = (key, value)
-        cache[name] = hit
-    return hit[1]
+    """One derived weight, ``build(*sources)``, cached as ``cached_value`` does."""
+    return cached_value(module, name, sources, lambda: build(*sources).contiguous())
 
 
 def _bf16(*ws):
@@ -582,12 +585,11 @@ def trimul(module, x, mask, outgoing, out_mode=OUT_BF16, out=None, workspace=Non
     _check(mask.shape == x.shape[:2] and mask.dtype == torch.float32 and mask.is_contiguous(),
            "expected a contiguous fp32 [N, N] mask")
     n = x.size(0)
-    w_in = cached_weight(module, "w_in", (module.p_in.weight, module.g_in.weight), _bf16)
-    w_pout = cached_weight(module, "w_pout", (module.p_out.weight,), _bf16)
-    w_gout = cached_weight(module, "w_gout", (module.g_out.weight,), _bf16)
     ni, no = module.norm_in, module.norm_out
-    niw, nib = cached_weight(module, "ni_w", (ni.weight,), _f32), cached_weight(module, "ni_b", (ni.bias,), _f32)
-    now, nob = cached_weight(module, "no_w", (no.weight,), _f32), cached_weight(module, "no_b", (no.bias,), _f32)
+    srcs = (module.p_in.weight, module.g_in.weight, module.p_out.weight, module.g_out.weight, ni.weight, ni.bias,
+            no.weight, no.bias)
+    w_in, w_pout, w_gout, niw, nib, now, nob = cached_value(module, "trimul", srcs, lambda: (
+        _bf16(*srcs[:2]), _bf16(srcs[2]), _bf16(srcs[3]), *map(_f32, srcs[4:])))
     out = _out_tensor(x, out, out_mode)
     rs = _row_scale(row_scale, x, n)
     nbytes = N.lib().bmx_trimul_workspace_bytes(n)
@@ -637,14 +639,11 @@ def triattn(module, x, mask, starting, out_mode=OUT_BF16, out=None, workspace=No
         _check(mask.shape == x.shape[:2] and mask.dtype == torch.float32 and mask.is_contiguous(),
                "expected a contiguous fp32 [N, N] mask")
     mha = module.mha
-    w_proj = cached_weight(module, "w_proj", (mha.linear_q.weight, mha.linear_k.weight, mha.linear_v.weight,
-                                              module.linear.weight), _triattn_proj_weight)
-    w_g = cached_weight(module, "w_g", (mha.linear_g.weight,), _bf16)
-    w_o = cached_weight(module, "w_o", (mha.linear_o.weight,), _bf16)
-    b_g = cached_weight(module, "b_g", (mha.linear_g.bias,), _f32)
-    b_o = cached_weight(module, "b_o", (mha.linear_o.bias,), _f32)
-    ln = module.layer_norm
-    lnw, lnb = cached_weight(module, "ln_w", (ln.weight,), _f32), cached_weight(module, "ln_b", (ln.bias,), _f32)
+    ln, lg, lo = module.layer_norm, mha.linear_g, mha.linear_o
+    srcs = (mha.linear_q.weight, mha.linear_k.weight, mha.linear_v.weight, module.linear.weight, lg.weight, lo.weight,
+            lg.bias, lo.bias, ln.weight, ln.bias)
+    w_proj, w_g, w_o, b_g, b_o, lnw, lnb = cached_value(module, "triattn", srcs, lambda: (
+        _triattn_proj_weight(*srcs[:4]), _bf16(srcs[4]), _bf16(srcs[5]), *map(_f32, srcs[6:])))
     out = _out_tensor(x, out, out_mode)
     rs = _row_scale(row_scale, x, n)
     nbytes = N.lib().bmx_triattn_workspace_bytes(n)
@@ -830,18 +829,18 @@ def pair_transition(module, x, out_mode=OUT_BF16, out=None, pair_bias=None):
     _cuda(x)
     _check(x.shape[-1] == C and x.dtype in (torch.float32, torch.bfloat16) and x.is_contiguous(),
            "expected contiguous fp32/bf16 x with 128 channels")
-    _check(module.fc1.weight.shape == (4 * C, C) and module.fc3.weight.shape == (C, 4 * C),
-           "expected a 128 -> 512 -> 128 transition")
-    w12 = cached_weight(module, "w12p", (module.fc1.weight, module.fc2.weight), _bf16_packed)
-    w3 = cached_weight(module, "w3p", (module.fc3.weight,), _bf16_packed)
-    lnw = cached_weight(module, "ln_w", (module.norm.weight,), _f32)
-    lnb = cached_weight(module, "ln_b", (module.norm.bias,), _f32)
+    fc1, fc3 = module.fc1.weight, module.fc3.weight
+    _check(fc1.shape == (4 * C, C) and fc3.shape == (C, 4 * C), "expected a 128 -> 512 -> 128 transition")
+    ln = module.norm
+    srcs = (fc1, module.fc2.weight, fc3, ln.weight, ln.bias)
+    w12, w3, lnw, lnb = cached_value(module, "transition", srcs, lambda: (
+        _bf16_packed(*srcs[:2]), _bf16_packed(srcs[2]), _f32(srcs[3]), _f32(srcs[4])))
     out = _out_tensor(x, out, out_mode)
     rows = x.numel() // C
     if pair_bias is None:
         if rows:
             N.call("bmx_pair_transition_fwd", x.data_ptr(), _code(x.dtype), rows, lnw.data_ptr(), lnb.data_ptr(),
-                   float(module.norm.eps), w12.data_ptr(), w3.data_ptr(), out.data_ptr(), out_mode, _stream(x))
+                   float(ln.eps), w12.data_ptr(), w3.data_ptr(), out.data_ptr(), out_mode, _stream(x))
         return out
     norm, lin, bias_out = pair_bias
     _check(out_mode != OUT_BF16, "the fused pair bias needs an fp32 out_mode")
@@ -851,7 +850,7 @@ def pair_transition(module, x, out_mode=OUT_BF16, out=None, pair_bias=None):
     fold = cached_weight(lin, "pair_bias_fold", (norm.weight, norm.bias, lin.weight), pair_bias_fold)
     if rows:
         N.call("bmx_pair_transition_bias_fwd", x.data_ptr(), _code(x.dtype), rows, lnw.data_ptr(), lnb.data_ptr(),
-               float(module.norm.eps), w12.data_ptr(), w3.data_ptr(), out.data_ptr(), out_mode, fold.data_ptr(),
+               float(ln.eps), w12.data_ptr(), w3.data_ptr(), out.data_ptr(), out_mode, fold.data_ptr(),
                float(norm.eps), bias_out.data_ptr(), _stream(x))
     return out
 

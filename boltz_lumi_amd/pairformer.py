@@ -220,19 +220,22 @@ def sequence_ok(layer, s, z, mask) -> bool:
     AttentionPairBias of 16 heads x 24 over a 384-channel s of N tokens with an
     [B, N] mask, its proj_o without bias, a plain pre_norm_s."""
     att = getattr(layer, "attention", None)
-    return (att is not None and type(att).__name__ == "AttentionPairBias" and _plain(att) and "forward" not in vars(att)
-            and getattr(att, "num_heads", None) == 16 and getattr(att, "c_s", None) == 384
-            and all(_plain(m) and "forward" not in vars(m)
-                    for m in (att.proj_q, att.proj_k, att.proj_v, att.proj_g, att.proj_o))
-            and att.proj_o.bias is None and _plain(layer.pre_norm_s) and "forward" not in vars(layer.pre_norm_s)
+    if att is None or type(att).__name__ != "AttentionPairBias" or _own(att) is None:
+        return False
+    kids = att._modules
+    return (getattr(att, "num_heads", None) == 16 and getattr(att, "c_s", None) == 384
+            and all(_own(kids[name]) is not None for name in ("proj_q", "proj_k", "proj_v", "proj_g", "proj_o"))
+            and getattr(kids["proj_o"], "bias", None) is None and _own(layer.pre_norm_s) is not None
             and s is not None and s.dim() == 3 and s.shape[0] == z.shape[0] and s.shape[1] == z.shape[1]
             and s.shape[2] == 384 and s.device == z.device
             and mask is not None and tuple(mask.shape) == tuple(s.shape[:2]) and mask.device == z.device)
 
 
-def _layer_norm_384(norm) -> bool:
-    return (type(norm) is torch.nn.LayerNorm and _plain(norm) and "forward" not in vars(norm)
-            and tuple(norm.normalized_shape) == (384,) and norm.weight is not None and norm.bias is not None)
+def _own(module):
+    """``module``'s own parameters by name, or None where it is hooked or its
+    forward is replaced.  Children and parameters are read from nn.Module's
+    dicts here: its __getattr__ costs more than the checks."""
+    return None if not _plain(module) or "forward" in module.__dict__ else module._parameters
 
 
 def _native_sequence_params(layer, device):
@@ -240,24 +243,31 @@ def _native_sequence_params(layer, device):
     stack (``sequence_ok`` holds) may run as that one call: plain LayerNorms,
     an upstream Transition(384) without biases, unhooked, and fp32 contiguous
     parameters on ``device``; else None."""
-    att, tr = layer.attention, layer.transition_s
-    if not (type(tr).__name__ == "Transition" and _plain(tr) and "forward" not in vars(tr)
-            and _layer_norm_384(layer.pre_norm_s) and _layer_norm_384(tr.norm)
-            and all(_plain(m) and "forward" not in vars(m) for m in (tr.fc1, tr.fc2, tr.fc3))
-            and _no_bias(tr.fc1, tr.fc2, tr.fc3, att.proj_k, att.proj_v, att.proj_g, att.proj_o)
-            and type(getattr(tr, "silu", None)) is torch.nn.SiLU):
+    kids = layer._modules
+    att, tr, pre = kids["attention"], kids.get("transition_s"), kids["pre_norm_s"]
+    if type(tr).__name__ != "Transition" or _own(tr) is None or type(pre) is not torch.nn.LayerNorm:
         return None
-    hidden = tr.fc1.weight.shape[0]
-    if hidden % 32 or not (_shape(tr.fc1.weight, hidden, 384) and _shape(tr.fc2.weight, hidden, 384)
-                           and _shape(tr.fc3.weight, 384, hidden)
-                           and all(_shape(m.weight, 384, 384)
-                                   for m in (att.proj_q, att.proj_k, att.proj_v, att.proj_g, att.proj_o))):
+    tk, ak = tr._modules, att._modules
+    norm = tk.get("norm")
+    if type(norm) is not torch.nn.LayerNorm or type(tk.get("silu")) is not torch.nn.SiLU:
         return None
-    sources = (att.proj_q.weight, att.proj_k.weight, att.proj_v.weight, att.proj_g.weight, att.proj_o.weight,
-               tr.fc1.weight, tr.fc2.weight, tr.fc3.weight)
-    rest = (layer.pre_norm_s.weight, layer.pre_norm_s.bias, tr.norm.weight, tr.norm.bias)
-    if not fp32_contiguous_on(device, *sources, *rest, *(() if att.proj_q.bias is None else (att.proj_q.bias,))):
+    own = [_own(m) for m in (pre, norm, ak["proj_q"], ak["proj_k"], ak["proj_v"], ak["proj_g"], ak["proj_o"],
+                             tk["fc1"], tk["fc2"], tk["fc3"])]
+    if any(o is None or o.get("weight") is None for o in own):
         return None
+    if any(o.get("bias") is not None for o in own[3:]) or own[0].get("bias") is None or own[1].get("bias") is None:
+        return None
+    hidden = own[7]["weight"].shape[0]
+    shapes = [(384,), (384,)] + [(384, 384)] * 5 + [(hidden, 384), (hidden, 384), (384, hidden)]
+    weights = [o["weight"] for o in own]
+    rest = [weights[0], own[0]["bias"], weights[1], own[1]["bias"]]
+    q_bias = own[2].get("bias")
+    sources = weights[2:]
+    if hidden % 32 or any(w.shape != shape for w, shape in zip(weights, shapes)):
+        return None
+    for p in sources + rest + ([] if q_bias is None else [q_bias]):
+        if p.dtype != torch.float32 or not p.is_contiguous() or p.device != device:
+            return None
 
     def build():
         q, k, v, g, o, fc1, fc2, fc3 = sources
@@ -266,7 +276,7 @@ def _native_sequence_params(layer, device):
                 ops.f32_pack(384, hidden, (0, 1, fc3)))
 
     qkvg, o, up, down = ops.cached_value(layer, "sequence_pack", sources, build)
-    return rest[0], rest[1], qkvg, att.proj_q.bias, o, rest[2], rest[3], up, down
+    return (rest[0], rest[1], qkvg, q_bias, o, rest[2], rest[3], up, down), hidden
 
 
 def sequence_stack(layer, s, z, mask, pair_bias=None):
@@ -283,10 +293,10 @@ def sequence_stack(layer, s, z, mask, pair_bias=None):
                 and not layer.training and s.shape[0] > 0 and s.shape[1] > 0):
             params = _native_sequence_params(layer, s.device)
             if params is not None:
-                tr, m = layer.transition_s, mask.float()
-                s = ops.sequence_stack(s.contiguous(), params, layer.pre_norm_s.eps, tr.norm.eps, pair_bias,
-                                       m if m.stride(1) == 1 else m.contiguous(), layer.attention.num_heads,
-                                       tr.fc1.weight.shape[0], layer.attention.inf)
+                m, att = mask.float(), layer.attention
+                s = ops.sequence_stack(s.contiguous(), params[0], layer.pre_norm_s.eps, layer.transition_s.norm.eps,
+                                       pair_bias, m if m.stride(1) == 1 else m.contiguous(), att.num_heads, params[1],
+                                       att.inf)
                 return layer.s_post_norm(s)
         s_normed = layer.pre_norm_s(s)
         o = None
