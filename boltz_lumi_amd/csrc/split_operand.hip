@@ -36,7 +36,7 @@ using namespace bmx;
 namespace {
 
 constexpr int kTail = 64;       // operand columns past 3 k
-constexpr int kRowChunks = 4;   // float4 chunks per lane for the LayerNorm passes: rows of <= 1024 values
+constexpr int kRowChunks = 4;   // most float4 chunks per lane for the LayerNorm passes: rows of <= 1024 values
 
 __device__ __forceinline__ void put_split(bf16* row, int64_t k, int64_t col, f32x4 v) {
   bf16x4 hi, lo;
@@ -89,75 +89,85 @@ __global__ __launch_bounds__(256) void split3_kernel(const float* __restrict__ x
   o.tail(lane);
 }
 
-// Row statistics of LayerNorm over d values held as float4 chunks
-// lane + 64 u (u < kRowChunks): the two-pass mean / biased variance of the
+// The LayerNorm passes hold a row as float4 chunks lane + L u (u < U) of L
+// lanes: a wave per row with U = 4 chunks a lane up to 1024 values, half a wave
+// with one chunk up to 128 (the atom transformer's rows: a whole wave left half
+// its lanes idle and loaded every operand four times over, 40960 x 128: residual
+// + AdaLN 47.7 us against 27.3, AdaLN 31.4 against 18.6).
+template <int L>
+__device__ __forceinline__ float row_sum(float v) {
+  return L == kWave ? wave_sum_full(v) : half_sum(v);
+}
+
+// Row statistics of LayerNorm: the two-pass mean / biased variance of the
 // LayerNorm kernels in norm.hip, same summation order.
 struct RowNorm {
   float mean, inv;
 };
-__device__ __forceinline__ RowNorm row_norm(const f32x4 (&v)[kRowChunks], int lane, int chunks, int d, float eps) {
+template <int L, int U>
+__device__ __forceinline__ RowNorm row_norm(const f32x4 (&v)[U], int lane, int chunks, int d, float eps) {
 #pragma clang fp contract(off)
   float s = 0.f;
 #pragma unroll
-  for (int u = 0; u < kRowChunks; ++u)
-    if (lane + kWave * u < chunks) s += v[u][0] + v[u][1] + v[u][2] + v[u][3];
-  const float mean = wave_sum_full(s) / d;
+  for (int u = 0; u < U; ++u)
+    if (lane + L * u < chunks) s += v[u][0] + v[u][1] + v[u][2] + v[u][3];
+  const float mean = row_sum<L>(s) / d;
   float q = 0.f;
 #pragma unroll
-  for (int u = 0; u < kRowChunks; ++u) {
-    if (lane + kWave * u < chunks) {
+  for (int u = 0; u < U; ++u) {
+    if (lane + L * u < chunks) {
       const f32x4 dv = v[u] - mean;
       q += dv[0] * dv[0] + dv[1] * dv[1] + dv[2] * dv[2] + dv[3] * dv[3];
     }
   }
-  return RowNorm{mean, rsqrtf(wave_sum_full(q) / d + eps)};
+  return RowNorm{mean, rsqrtf(row_sum<L>(q) / d + eps)};
 }
 
 // tn > 0: the rows of x are the pairs of a tn x tn frame read transposed
 // (operand row i tn + j is x row j tn + i).
-template <bool PACKED>
+template <bool PACKED, int L, int U>
 __global__ __launch_bounds__(256) void layernorm_split3_kernel(const float* __restrict__ x, int64_t ldx,
                                                                bf16* __restrict__ out, int64_t rows, int d,
                                                                float eps, int64_t tn) {
 #pragma clang fp contract(off)
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t row = (int64_t)blockIdx.x * (256 / L) + threadIdx.x / L;
   if (row >= rows) return;
-  const int lane = threadIdx.x & 63, chunks = d >> 2;
+  const int lane = threadIdx.x % L, chunks = d >> 2;
   const float* xr = x + (tn ? (row % tn) * tn + row / tn : row) * ldx;
-  f32x4 v[kRowChunks];
+  f32x4 v[U];
 #pragma unroll
-  for (int u = 0; u < kRowChunks; ++u) v[u] = load4(xr + 4 * min(lane + kWave * u, chunks - 1));
-  const RowNorm n = row_norm(v, lane, chunks, d, eps);
+  for (int u = 0; u < U; ++u) v[u] = load4(xr + 4 * min(lane + L * u, chunks - 1));
+  const RowNorm n = row_norm<L>(v, lane, chunks, d, eps);
   const OperandRow<PACKED> o(out, row, d);
 #pragma unroll
-  for (int u = 0; u < kRowChunks; ++u)
-    if (lane + kWave * u < chunks) o.put(4 * (lane + kWave * u), (v[u] - n.mean) * n.inv);
+  for (int u = 0; u < U; ++u)
+    if (lane + L * u < chunks) o.put(4 * (lane + L * u), (v[u] - n.mean) * n.inv);
   o.tail(lane);
 }
 
 // sigmoid(scale) * LN(a) + shift as bmx_adaln rounds it (the product and the
 // sum separately), scale and shift rows at stride ldm.
-template <bool PACKED>
+template <bool PACKED, int L, int U>
 __global__ __launch_bounds__(256) void adaln_split3_kernel(const float* __restrict__ a, const float* __restrict__ scale,
                                                            const float* __restrict__ shift, int64_t ldm,
                                                            bf16* __restrict__ out, int64_t rows, int d, float eps) {
 #pragma clang fp contract(off)
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t row = (int64_t)blockIdx.x * (256 / L) + threadIdx.x / L;
   if (row >= rows) return;
-  const int lane = threadIdx.x & 63, chunks = d >> 2;
-  f32x4 v[kRowChunks], sc[kRowChunks], sh[kRowChunks];
+  const int lane = threadIdx.x % L, chunks = d >> 2;
+  f32x4 v[U], sc[U], sh[U];
 #pragma unroll
-  for (int u = 0; u < kRowChunks; ++u) {
-    const int c = 4 * min(lane + kWave * u, chunks - 1);
+  for (int u = 0; u < U; ++u) {
+    const int c = 4 * min(lane + L * u, chunks - 1);
     v[u] = load4(a + row * d + c);
     sc[u] = load4(scale + row * ldm + c);
     sh[u] = load4(shift + row * ldm + c);
   }
-  const RowNorm n = row_norm(v, lane, chunks, d, eps);
+  const RowNorm n = row_norm<L>(v, lane, chunks, d, eps);
   const OperandRow<PACKED> o(out, row, d);
 #pragma unroll
-  for (int u = 0; u < kRowChunks; ++u) {
-    if (lane + kWave * u < chunks) {
+  for (int u = 0; u < U; ++u) {
+    if (lane + L * u < chunks) {
       f32x4 r;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -165,7 +175,7 @@ __global__ __launch_bounds__(256) void adaln_split3_kernel(const float* __restri
         const float prod = sigmoid_f(sc[u][e]) * an;
         r[e] = prod + sh[u][e];
       }
-      o.put(4 * (lane + kWave * u), r);
+      o.put(4 * (lane + L * u), r);
     }
   }
   o.tail(lane);
@@ -175,19 +185,19 @@ __global__ __launch_bounds__(256) void adaln_split3_kernel(const float* __restri
 // r = c + sigmoid(g) * a (the MODULATION epilogue; g and the modulation rows at
 // strides ldg / ldm) is written to out (which may alias c), then the operand
 // row of sigmoid(scale) * LN(r) + shift, rounded as bmx_adaln_split3_bf16.
-template <bool PACKED>
+template <bool PACKED, int L, int U>
 __global__ __launch_bounds__(256) void gated_residual_adaln_split3_kernel(
     const float* __restrict__ a, const float* __restrict__ g, int64_t ldg, const float* c, float* out,
     const float* __restrict__ scale, const float* __restrict__ shift, int64_t ldm, bf16* __restrict__ op,
     int64_t rows, int d, float eps) {
 #pragma clang fp contract(off)
-  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t row = (int64_t)blockIdx.x * (256 / L) + threadIdx.x / L;
   if (row >= rows) return;
-  const int lane = threadIdx.x & 63, chunks = d >> 2;
-  f32x4 v[kRowChunks], sc[kRowChunks], sh[kRowChunks];
+  const int lane = threadIdx.x % L, chunks = d >> 2;
+  f32x4 v[U], sc[U], sh[U];
 #pragma unroll
-  for (int u = 0; u < kRowChunks; ++u) {
-    const int col = 4 * min(lane + kWave * u, chunks - 1);
+  for (int u = 0; u < U; ++u) {
+    const int col = 4 * min(lane + L * u, chunks - 1);
     const f32x4 av = load4(a + row * d + col), gv = load4(g + row * ldg + col), cv = load4(c + row * d + col);
     sc[u] = load4(scale + row * ldm + col);
     sh[u] = load4(shift + row * ldm + col);
@@ -198,13 +208,13 @@ __global__ __launch_bounds__(256) void gated_residual_adaln_split3_kernel(
     }
   }
 #pragma unroll
-  for (int u = 0; u < kRowChunks; ++u)
-    if (lane + kWave * u < chunks) store4(out + row * d + 4 * (lane + kWave * u), v[u]);
-  const RowNorm n = row_norm(v, lane, chunks, d, eps);
+  for (int u = 0; u < U; ++u)
+    if (lane + L * u < chunks) store4(out + row * d + 4 * (lane + L * u), v[u]);
+  const RowNorm n = row_norm<L>(v, lane, chunks, d, eps);
   const OperandRow<PACKED> o(op, row, d);
 #pragma unroll
-  for (int u = 0; u < kRowChunks; ++u) {
-    if (lane + kWave * u < chunks) {
+  for (int u = 0; u < U; ++u) {
+    if (lane + L * u < chunks) {
       f32x4 r;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -212,7 +222,7 @@ __global__ __launch_bounds__(256) void gated_residual_adaln_split3_kernel(
         const float prod = sigmoid_f(sc[u][e]) * an;
         r[e] = prod + sh[u][e];
       }
-      o.put(4 * (lane + kWave * u), r);
+      o.put(4 * (lane + L * u), r);
     }
   }
   o.tail(lane);
@@ -245,6 +255,16 @@ __global__ __launch_bounds__(256) void swiglu_split3_kernel(const float* __restr
 
 inline unsigned row_blocks(int64_t rows) { return (unsigned)((rows + 3) / 4); }
 
+// Launch of a LayerNorm pass over rows of d values: half a wave per row up to
+// 128 values, a wave above.
+#define ROW_LAUNCH(kernel, packed, ...)                                                                \
+  do {                                                                                                 \
+    if (d <= 128)                                                                                      \
+      kernel<packed, 32, 1><<<(unsigned)((rows + 7) / 8), 256, 0, stream>>>(__VA_ARGS__);              \
+    else                                                                                               \
+      kernel<packed, kWave, kRowChunks><<<row_blocks(rows), 256, 0, stream>>>(__VA_ARGS__);            \
+  } while (0)
+
 }  // namespace
 
 namespace bmx {
@@ -255,21 +275,20 @@ int split_packed(const float* x, int64_t rows, int d, bf16* op, hipStream_t stre
 }
 
 int layernorm_packed(const float* x, int64_t rows, int d, float eps, bf16* op, hipStream_t stream) {
-  layernorm_split3_kernel<true><<<row_blocks(rows), 256, 0, stream>>>(x, d, op, rows, d, eps, 0);
+  ROW_LAUNCH(layernorm_split3_kernel, true, x, d, op, rows, d, eps, 0);
   return check_launch("layernorm_packed");
 }
 
 int adaln_packed(const float* a, const float* scale, const float* shift, int64_t ldm, int64_t rows, int d, float eps,
                  bf16* op, hipStream_t stream) {
-  adaln_split3_kernel<true><<<row_blocks(rows), 256, 0, stream>>>(a, scale, shift, ldm, op, rows, d, eps);
+  ROW_LAUNCH(adaln_split3_kernel, true, a, scale, shift, ldm, op, rows, d, eps);
   return check_launch("adaln_packed");
 }
 
 int gated_residual_adaln_packed(const float* a, const float* g, int64_t ldg, const float* c, float* out,
                                 const float* scale, const float* shift, int64_t ldm, int64_t rows, int d, float eps,
                                 bf16* op, hipStream_t stream) {
-  gated_residual_adaln_split3_kernel<true>
-      <<<row_blocks(rows), 256, 0, stream>>>(a, g, ldg, c, out, scale, shift, ldm, op, rows, d, eps);
+  ROW_LAUNCH(gated_residual_adaln_split3_kernel, true, a, g, ldg, c, out, scale, shift, ldm, op, rows, d, eps);
   return check_launch("gated_residual_adaln_packed");
 }
 
@@ -299,7 +318,8 @@ int bmx_layernorm_split3_bf16(const float* x, int64_t rows, int dim, int64_t ldx
   BMX_REQUIRE(x && out, "bmx_layernorm_split3_bf16: null pointer");
   BMX_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)out % 8 == 0,
               "bmx_layernorm_split3_bf16: x must be 16-byte and out 8-byte aligned");
-  layernorm_split3_kernel<false><<<row_blocks(rows), 256, 0, stream>>>(x, ldx, (bf16*)out, rows, dim, eps, 0);
+  const int d = dim;
+  ROW_LAUNCH(layernorm_split3_kernel, false, x, ldx, (bf16*)out, rows, d, eps, 0);
   return check_launch("bmx_layernorm_split3_bf16");
 }
 
@@ -313,7 +333,9 @@ int bmx_layernorm_split3_t_bf16(const float* x, int64_t n, int dim, int64_t ldx,
   BMX_REQUIRE(x && out, "bmx_layernorm_split3_t_bf16: null pointer");
   BMX_REQUIRE((uintptr_t)x % 16 == 0 && (uintptr_t)out % 8 == 0,
               "bmx_layernorm_split3_t_bf16: x must be 16-byte and out 8-byte aligned");
-  layernorm_split3_kernel<false><<<row_blocks(n * n), 256, 0, stream>>>(x, ldx, (bf16*)out, n * n, dim, eps, n);
+  const int d = dim;
+  const int64_t rows = n * n;
+  ROW_LAUNCH(layernorm_split3_kernel, false, x, ldx, (bf16*)out, rows, d, eps, n);
   return check_launch("bmx_layernorm_split3_t_bf16");
 }
 
@@ -328,7 +350,8 @@ int bmx_adaln_split3_bf16(const float* a, const float* scale, const float* shift
   BMX_REQUIRE(a && scale && shift && out, "bmx_adaln_split3_bf16: null pointer");
   BMX_REQUIRE(((uintptr_t)a | (uintptr_t)scale | (uintptr_t)shift) % 16 == 0 && (uintptr_t)out % 8 == 0,
               "bmx_adaln_split3_bf16: a, scale, shift must be 16-byte and out 8-byte aligned");
-  adaln_split3_kernel<false><<<row_blocks(rows), 256, 0, stream>>>(a, scale, shift, ld_mod, (bf16*)out, rows, dim, eps);
+  const int d = dim;
+  ROW_LAUNCH(adaln_split3_kernel, false, a, scale, shift, ld_mod, (bf16*)out, rows, d, eps);
   return check_launch("bmx_adaln_split3_bf16");
 }
 
@@ -347,8 +370,8 @@ int bmx_gated_residual_adaln_split3_bf16(const float* a, const float* gate, int6
                       16 == 0 &&
                   (uintptr_t)op % 8 == 0,
               "bmx_gated_residual_adaln_split3_bf16: fp32 operands must be 16-byte and op 8-byte aligned");
-  gated_residual_adaln_split3_kernel<false><<<row_blocks(rows), 256, 0, stream>>>(a, gate, ld_gate, c, out, scale, shift,
-                                                                           ld_mod, (bf16*)op, rows, dim, eps);
+  const int d = dim;
+  ROW_LAUNCH(gated_residual_adaln_split3_kernel, false, a, gate, ld_gate, c, out, scale, shift, ld_mod, (bf16*)op, rows, d, eps);
   return check_launch("bmx_gated_residual_adaln_split3_bf16");
 }
 
