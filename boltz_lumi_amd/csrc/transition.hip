@@ -15,15 +15,15 @@ using namespace bmx;
 
 namespace {
 
-constexpr int kTP = 128, kHidden = 512;
+constexpr int kHidden = 512;
 
-// Write the 128 x 128 result tile held as y[nt] (D[pair][out], lane -> output
+// Write the TP x 128 result tile held as y[nt] (D[pair][out], lane -> output
 // channel, register r -> pair nt*32 + drow(r, lane)).  Residual modes load
-// all 64 base values before the first store: interleaving each load with the
+// all TP / 2 base values before the first store: interleaving each load with the
 // previous store would serialise them on the possible out / x alias.  FULL
 // tiles skip the row checks; the last tile clamps loads and masks stores.
-template <bool FULL, typename TIn>
-__device__ __forceinline__ void store_tile(f32x16 (&y)[4], const TIn* x, void* out, const float* base, int out_mode,
+template <bool FULL, int NT, typename TIn>
+__device__ __forceinline__ void store_tile(f32x16 (&y)[NT], const TIn* x, void* out, const float* base, int out_mode,
                                            int64_t r0, int64_t rows) {
   const int l = lane_id();
   const int64_t lane_off = base - (const float*)out;  // row (r0 + 4 h) * kC + channel
@@ -35,17 +35,17 @@ __device__ __forceinline__ void store_tile(f32x16 (&y)[4], const TIn* x, void* o
   };
   if (out_mode == kOutAccumulate) {
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) y[nt][r] += ((const float*)out)[offset(nt, r)];
   } else if (out_mode == kOutResidual) {
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) y[nt][r] += (float)x[offset(nt, r)];
   }
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt)
+  for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       if (!FULL && r0 + nt * 32 + drow(r, l) >= rows) continue;
@@ -78,13 +78,12 @@ constexpr size_t kFoldBytes = 2 * kFoldHalf * sizeof(bf16) + 16 * sizeof(float);
 
 constexpr int kZRow = kC + 8;  // fp32 LDS row of the updated tile: 4 rows apart = 32 banks apart
 
-// Row p of the tile's 128 updated fp32 rows: rows 0..63 over xn, 64..127 over hid.
-__device__ __forceinline__ float* zrow(bf16* xn, bf16* hid, int p) {
-  return (float*)(p < 64 ? xn : hid) + (p & 63) * kZRow;
-}
+// Row p of the tile's updated fp32 rows, over the xn and hid tiles (adjacent:
+// TP fp32 rows fill them exactly).
+__device__ __forceinline__ float* zrow(bf16* smem, int p) { return (float*)smem + p * kZRow; }
 
-// The rows are never normalised in place.  Wave w takes rows 32w .. 32w+31
-// as two 16-row tiles; lane (row l%16, group g) reads channels 32q + 8g .. +7
+// The rows are never normalised in place.  Wave w takes the 16-row tiles w, w +
+// 4, ...; lane (row l%16, group g) reads channels 32q + 8g .. +7
 // of its row (two 16-byte LDS loads per k step q); mu and the centred
 // variance come from in-lane sums and the xor-16 / xor-32 exchanges.  The
 // 128 -> 16 product runs on bf16 MFMA (16x16x32) with both operands split
@@ -123,12 +122,14 @@ __device__ __forceinline__ PairBiasFrags load_pair_bias_frags(const bf16* fold) 
   return f;
 }
 
-__device__ __forceinline__ void pair_bias_epilogue(bf16* xn, bf16* hid, const PairBiasFrags& f,
-                                                   const PairBiasArgs& pb, int64_t r0, int64_t rows) {
+template <int TP>
+__device__ __forceinline__ void pair_bias_epilogue(bf16* smem, const PairBiasFrags& f, const PairBiasArgs& pb,
+                                                   int64_t r0, int64_t rows) {
   const int l = lane_id(), w = threadIdx.x >> 6, g = l >> 4, hc = l & 15;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const float* row = zrow(xn, hid, 32 * w + 16 * j + hc) + 8 * g;
+  for (int j = 0; j < (TP + 63) / 64; ++j) {
+    if (TP < 64 && 16 * w >= TP) break;  // wave-uniform
+    const float* row = zrow(smem, 16 * (w + 4 * j) + hc) + 8 * g;
     f32x4 xv[8];
 #pragma unroll
     for (int q = 0; q < 4; ++q) xv[2 * q] = *(const f32x4*)(row + 32 * q), xv[2 * q + 1] = *(const f32x4*)(row + 32 * q + 4);
@@ -153,7 +154,7 @@ __device__ __forceinline__ void pair_bias_epilogue(bf16* xn, bf16* hid, const Pa
       acc1 = mfma16bf(f.wl[q], xh, acc1);
       acc1 = mfma16bf(f.wh[q], xl, acc1);
     }
-    const int64_t grow = r0 + 32 * w + 16 * j + hc;
+    const int64_t grow = r0 + 16 * (w + 4 * j) + hc;
     if (grow < rows) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) pb.out[(int64_t)(4 * g + r) * rows + grow] = fmaf(rstd, acc0[r] + acc1[r], f.bo[r]);
@@ -180,16 +181,20 @@ __global__ __launch_bounds__(256) void pair_bias_fold_kernel(const float* __rest
   }
 }
 
-template <typename TIn, bool BIAS>
+// TP rows per block.  128 rows per block read the 384 KB of packed weights
+// least often; with fewer rows than that fills the chip with, smaller tiles
+// (32 or 64 rows) take the same chain of phases on less work each.
+template <typename TIn, bool BIAS, int TP>
 __global__ __launch_bounds__(256, 2) void pair_transition_kernel(const TIn* x, const float* __restrict__ ln_w,
                                                               const float* __restrict__ ln_b, float eps,
                                                               const bf16* __restrict__ w12,
                                                               const bf16* __restrict__ w3, void* out, int out_mode,
                                                               int64_t rows, PairBiasArgs pb) {
-  __shared__ __attribute__((aligned(16))) bf16 xn[kTP * kLdsRow];
-  __shared__ __attribute__((aligned(16))) bf16 hid[kTP * kLdsRow];
-  static_assert(2 * kLdsRow * sizeof(bf16) == kZRow * sizeof(float), "64 fp32 rows must fit xn, 64 hid");
-  const int64_t r0 = (int64_t)blockIdx.x * kTP;
+  constexpr int NT = TP / 32;
+  __shared__ __attribute__((aligned(16))) bf16 smem[2 * TP * kLdsRow];
+  bf16 *xn = smem, *hid = smem + TP * kLdsRow;
+  static_assert(2 * kLdsRow * sizeof(bf16) == kZRow * sizeof(float), "TP fp32 rows must fill xn and hid");
+  const int64_t r0 = (int64_t)blockIdx.x * TP;
   const int t = threadIdx.x, l = lane_id(), w = t >> 6;
   const int c0 = 32 * w;  // this wave's 32 hidden channels of each chunk / 32 output channels
   // fc1 / fc2 rows of one 128-wide hidden chunk (A operands).  Chunk 0 is
@@ -206,16 +211,18 @@ __global__ __launch_bounds__(256, 2) void pair_transition_kernel(const TIn* x, c
   };
   load_w12(0);
   auto row_ptr = [&](int p) -> const TIn* { return r0 + p < rows ? x + (r0 + p) * kC : nullptr; };
-  ln_rows_to_lds<kTP, TIn>(row_ptr, x + r0 * kC, ln_w, ln_b, eps, xn);
+  ln_rows_to_lds<TP, TIn>(row_ptr, x + r0 * kC, ln_w, ln_b, eps, xn);
   __syncthreads();
 
-  f32x16 y[4] = {zero16(), zero16(), zero16(), zero16()};
+  f32x16 y[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) y[nt] = zero16();
   for (int hc = 0; hc < kHidden / kC; ++hc) {
     bf16x8 f3[8];
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) f3[ks] = pfrag(w3, kHidden, c0, 8 * hc + ks);
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
+    for (int nt = 0; nt < NT; ++nt) {
       f32x16 a1 = zero16(), a2 = zero16();
 #pragma unroll
       for (int ks = 0; ks < 8; ++ks) {
@@ -223,7 +230,7 @@ __global__ __launch_bounds__(256, 2) void pair_transition_kernel(const TIn* x, c
         a1 = mfma32(f1[ks], xf, a1);
         a2 = mfma32(f2[ks], xf, a2);
       }
-      if (nt == 3 && hc + 1 < kHidden / kC) load_w12(hc + 1);
+      if (nt == NT - 1 && hc + 1 < kHidden / kC) load_w12(hc + 1);
       // D[hidden][pair]: lane -> pair nt*32 + l%32, registers 4q..4q+3 ->
       // hidden channels c0 + 8q + 4(l/32) + 0..3, stored as one 8-byte write.
       bf16* dst = hid + (nt * 32 + (l & 31)) * kLdsRow + c0 + 4 * (l >> 5);
@@ -237,7 +244,7 @@ __global__ __launch_bounds__(256, 2) void pair_transition_kernel(const TIn* x, c
     }
     __syncthreads();
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int ks = 0; ks < 8; ++ks) y[nt] = mfma32(frag(hid, kLdsRow, nt * 32, ks), f3[ks], y[nt]);
     __syncthreads();
@@ -245,13 +252,13 @@ __global__ __launch_bounds__(256, 2) void pair_transition_kernel(const TIn* x, c
   // D[pair][out]: lane -> output channel c0 + l%32, register r -> pair
   // nt*32 + drow(r, l).
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt)
+  for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) y[nt][r] = rbf(y[nt][r]);
   const float* base = (const float*)out + (r0 + 4 * (l >> 5)) * kC + c0 + (l & 31);
   PairBiasFrags pbf;
   if constexpr (BIAS) pbf = load_pair_bias_frags(pb.fold);
-  if (r0 + kTP <= rows)
+  if (r0 + TP <= rows)
     store_tile<true>(y, x, out, base, out_mode, r0, rows);
   else
     store_tile<false>(y, x, out, base, out_mode, r0, rows);
@@ -259,11 +266,11 @@ __global__ __launch_bounds__(256, 2) void pair_transition_kernel(const TIn* x, c
     // y now holds the stored fp32 rows (residual included); the loop's last
     // barrier has released xn / hid.
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) zrow(xn, hid, nt * 32 + drow(r, l))[c0 + (l & 31)] = y[nt][r];
+      for (int r = 0; r < 16; ++r) zrow(smem, nt * 32 + drow(r, l))[c0 + (l & 31)] = y[nt][r];
     __syncthreads();
-    pair_bias_epilogue(xn, hid, pbf, pb, r0, rows);
+    pair_bias_epilogue<TP>(smem, pbf, pb, r0, rows);
   }
 }
 
@@ -271,14 +278,30 @@ template <bool BIAS>
 int launch_transition(const char* name, const void* x, int x_dtype, int64_t rows, const float* ln_w,
                       const float* ln_b, float eps, const void* w12, const void* w3, void* out, int out_mode,
                       const PairBiasArgs& pb, hipStream_t stream) {
-  const unsigned grid = (unsigned)((rows + kTP - 1) / kTP);
+  auto go = [&](auto in, auto tp) {
+    using TIn = decltype(in);
+    constexpr int TP = decltype(tp)::value;
+    const unsigned grid = (unsigned)((rows + TP - 1) / TP);
+    pair_transition_kernel<TIn, BIAS, TP><<<grid, 256, 0, stream>>>((const TIn*)x, ln_w, ln_b, eps, (const bf16*)w12,
+                                                                    (const bf16*)w3, out, out_mode, rows, pb);
+  };
+  // The smallest tile that still runs in one round of two blocks per CU: below
+  // that the time is one block's chain of phases, which shortens with its rows
+  // (20^2 rows 19.8 -> 9.3 us, 117^2 20.9 -> 12.5 in 32-row tiles, 150^2 21.2 ->
+  // 17.3 in 64-row ones); above it 128-row tiles stream the weights least often.
+  const int64_t slots = 2 * device_cu_count();
+  auto pick = [&](auto in) {
+    if (rows <= 32 * slots)
+      go(in, std::integral_constant<int, 32>{});
+    else if (rows <= 64 * slots)
+      go(in, std::integral_constant<int, 64>{});
+    else
+      go(in, std::integral_constant<int, 128>{});
+  };
   if (x_dtype == kF32)
-    pair_transition_kernel<float, BIAS><<<grid, 256, 0, stream>>>((const float*)x, ln_w, ln_b, eps,
-                                                                  (const bf16*)w12, (const bf16*)w3, out, out_mode,
-                                                                  rows, pb);
+    pick(float{});
   else
-    pair_transition_kernel<bf16, BIAS><<<grid, 256, 0, stream>>>((const bf16*)x, ln_w, ln_b, eps, (const bf16*)w12,
-                                                                 (const bf16*)w3, out, out_mode, rows, pb);
+    pick(bf16{});
   return check_launch(name);
 }
 
