@@ -341,13 +341,6 @@ int token_attention_packed(const float* proj, int64_t batch, int64_t n, int head
 // packed fp32 operand (f32_packed_index) of batch * n rows.
 int sequence_attention_packed(const float* proj, int64_t batch, int64_t n, int heads, int head_dim, const float* bias,
                               const float* mask, int64_t smask, float inf, float* op, hipStream_t stream);
-// The split-bf16 attention on K / V^T already split and laid out as its pre-pass
-// writes them, n queries and n keys per element, elements b / bias_div sharing
-// dense bias [heads][n][n].
-int seq_attention_x3_presplit(const char* name, const float* q, const float* g, int64_t ldq, int64_t sq, int64_t batch,
-                              int64_t n, int heads, int head_dim, const float* bias, int64_t bias_div, const bf16* kh,
-                              const bf16* kl, const bf16* vth, const bf16* vtl, const float* mterm, float* out,
-                              hipStream_t stream);
 size_t token_attention_workspace(int64_t batch, int64_t n, int heads, int head_dim);
 }  // namespace bmx
 

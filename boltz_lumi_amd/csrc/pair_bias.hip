@@ -738,15 +738,6 @@ constexpr int64_t kX3MinKeys = 256;
 
 namespace bmx {
 
-int seq_attention_x3_presplit(const char* name, const float* q, const float* g, int64_t ldq, int64_t sq, int64_t batch,
-                              int64_t n, int heads, int head_dim, const float* bias, int64_t bias_div, const bf16* kh,
-                              const bf16* kl, const bf16* vth, const bf16* vtl, const float* mterm, float* out,
-                              hipStream_t stream) {
-  const SeqAttnShape sh{(int)n, (int)n, (int)bias_div, ldq, 0, sq, 0, heads * n * n, 0};
-  return launch_x3_attention(name, q, kh, kl, vth, vtl, mterm, bias, g, batch, sh, heads, head_dim, out, nullptr, false,
-                             stream);
-}
-
 size_t token_attention_workspace(int64_t batch, int64_t n, int heads, int head_dim) {
   return n >= kX3MinKeys ? x3_workspace_bytes(batch, n, heads, head_dim) : 0;
 }

@@ -709,10 +709,9 @@ def triattn_fp32(module, x, mask, starting, block_rows=None):
     q | k | v | g and the triangle bias with split-bf16 products (about 2^-16
     relative each) and writes the attention's operands
     (``bmx_triattn_fp32_fwd``; the ending node reads x's columns in place); the
-    attention, mask bias, softmax, PV product and gate run fused on the
-    split-bf16 kernel, every row i one batch element attending over its N keys,
-    all rows sharing the [4, N, N] triangle bias, so the [N, 4, N, N] scores
-    never reach HBM; ``linear_o`` is an fp32 GEMM.  In exact fp32 mode the fp32
+    attention, mask bias, softmax, PV product and gate run fused on split-bf16
+    products, two rows sharing each fetch of the [4, N, N] triangle bias, so the
+    [N, 4, N, N] scores never reach HBM; ``linear_o`` is an fp32 GEMM.  In exact fp32 mode the fp32
     LN128 kernel, fp32 GEMMs and the fp32-MFMA attention run instead.  Returns
     fp32 [N, N, 128].
 
@@ -755,7 +754,7 @@ def _triattn_fp32_split(module, x, mask, starting, rows):
     it for all rows)."""
     n, mha = x.shape[0], module.mha
     m = None if mask is None else mask.to(torch.float32).contiguous()
-    tri_bias = torch.empty(4, n, n, device=x.device, dtype=torch.float32)
+    tri_bias = torch.empty(4, n, (n + 63) // 64 * 64, device=x.device, dtype=torch.float32)
     ws = _workspace(N.lib().bmx_triattn_fp32_workspace_bytes(n, rows), x.device)
     w_o, b_o = mha.linear_o.weight.float(), mha.linear_o.bias.float()
     if rows >= n:
@@ -765,6 +764,7 @@ def _triattn_fp32_split(module, x, mask, starting, rows):
         del ws, tri_bias  # 2 KB per pair, before linear_o's output is allocated
         out = torch.nn.functional.linear(o, w_o, b_o)
     else:
+        rows -= rows % 2 if rows > 1 else 0  # the attention pairs rows: the pairs of one pass
         _triattn_fp32_native(module, x, m, starting, tri_bias, 1, 0, n)
         o = torch.empty(rows, n, C, device=x.device, dtype=torch.float32)
         out = torch.empty(n, n, C, device=x.device, dtype=torch.float32)  # the output frame

@@ -36,3 +36,26 @@ def test_fp32_projection_edges(gpu, n, starting, masked):
     assert (got - blocked).abs().max() / got.abs().max() < 1e-6
     err = ((got - want).abs().max() / want.abs().max()).item()
     assert err < 1e-4, err  # split products: 2^-16 relative each
+
+
+@pytest.mark.parametrize("n,scale,closed", [(97, 1.0, 70), (97, 1.0, 33), (130, 200.0, 0), (130, 200.0, 5), (1090, 1.0, 3)])
+def test_fp32_attention_offsets(gpu, n, scale, closed):
+    """The attention's shared offset comes from the first 32 keys: keys closed
+    before the open ones, scores far above the first keys' (a triangle bias of
+    hundreds), and more than one group of query tiles."""
+    g = torch.Generator().manual_seed(n + closed)
+    layer = R.randomize(R.TriangleAttention(128, 32, 4), generator=g).to(gpu).eval()
+    x = torch.randn(n, n, 128, generator=g).to(gpu)
+    with torch.no_grad():
+        layer.linear.weight.mul_(scale)
+    mask = torch.ones(n, n, device=gpu)
+    mask[::3, :closed] = 0
+    with torch.inference_mode():
+        got = ops.triattn_fp32(layer, x, mask, True)
+        want = layer(x[None], mask[None], chunk_size=64)[0]
+        top = layer.linear(layer.layer_norm(x)).abs().max().item()
+    err = ((got - want).abs().max() / want.abs().max()).item()
+    print(f"n={n} scale={scale} closed={closed}: largest bias {top:.1f}, error {err:.2e}", flush=True)
+    assert scale == 1.0 or top > 100
+    # split products: 2^-16 relative each; an error of a score is a relative error of its probability
+    assert err < max(1e-4, 2 * 2**-16 * top)
