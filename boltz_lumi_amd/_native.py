@@ -44,6 +44,7 @@ SIGNATURES = {
     "bmx_triattn_fp32_workspace_bytes": (c_size_t, [c_int64, c_int64]),
     "bmx_triattn_fp32_fwd": (c_int, [_P, _P, c_int64, c_int, c_int64, c_int64, c_float, _P, _P, c_float, _P, _P, _P, _P,
                                      c_int, _P, _P, c_size_t, _P]),
+    "bmx_linear128_f32_fwd": (c_int, [_P, c_int64, _P, _P, _P, _P]),
     "bmx_f32_pack": (c_int, [_P, c_int64, c_int64, c_int64, c_int64, c_int64, _P, _P]),
     "bmx_sequence_stack_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64]),
     "bmx_sequence_stack_fwd": (c_int, [_P, c_int64, c_int64, c_int, c_int, c_int64, _P, c_float, c_float, _P, _P, c_int64,

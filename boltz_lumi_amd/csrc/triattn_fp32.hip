@@ -514,6 +514,72 @@ __global__ __launch_bounds__(kCoreThreads) __attribute__((amdgpu_waves_per_eu(4)
   if (closed || !core_rows<true>(a, i0, h, qw, mask_k0, lds)) core_rows<false>(a, i0, h, qw, mask_k0, lds);
 }
 
+// ------------------------------------------------------------------ output linear
+// out = o W^T + b over rows of 128, fp32 MFMA (32x32x2).  Weight-stationary: wave w
+// keeps outputs 32 (w % 4) .. + 31 (64 VGPRs) and takes rows 32 (w / 4) .. + 31 of a
+// 64-row tile; the next tile comes by LDS DMA, 16-byte chunk c of row r at position
+// c ^ (r % 32).  Lane l holds chunk 2 j + l / 32 of its row for k step j, so MFMA e of a step
+// multiplies k = 8 j + e and 8 j + 4 + e; D[output][row] leaves as 16-byte stores.
+// What bounds it: the fp32 matrix cores (75 us of them at n = 576; 129 us).  The library GEMM took
+// 162-179 us.  out may be o: a block has read a tile when it writes it, and nobody else reads it.
+constexpr int kLinRows = 64, kLinWaves = 8, kLinTile = kLinRows * kC * 4;
+
+__global__ __launch_bounds__(64 * kLinWaves) __attribute__((amdgpu_waves_per_eu(4))) void linear128_f32_kernel(
+    const float* o, int64_t rows, const float* __restrict__ w_o, const float* __restrict__ b_o, float* out) {
+  __shared__ __attribute__((aligned(16))) char lds[2 * kLinTile];
+  __shared__ __attribute__((aligned(16))) float sbias[kC];
+  const int l = lane_id(), hh = l >> 5, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c0 = 32 * (w & 3), r0 = 32 * (w >> 2), row = r0 + (l & 31);
+  const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+  f32x4 wf[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) wf[j] = load4(w_o + (c0 + (l & 31)) * kC + 8 * j + 4 * hh);
+  if (threadIdx.x < kC) sbias[threadIdx.x] = b_o[threadIdx.x];
+  auto dma_tile = [&](int buf, int64_t tile) {
+#pragma unroll
+    for (int u = 0; u < kLinTile / 1024 / kLinWaves; ++u) {
+      const int piece = w + kLinWaves * u, r = 2 * piece + hh;  // 1 KB: two rows
+      const int64_t at = tile * kLinRows + r < rows ? tile * kLinRows + r : rows - 1;  // not stored past the end
+      lds_dma16(o + at * kC + 4 * ((l & 31) ^ (r & 31)),
+                __builtin_amdgcn_readfirstlane(lds0 + buf * kLinTile + 1024 * piece));
+    }
+  };
+  const int64_t tiles = (rows + kLinRows - 1) / kLinRows;
+  int64_t tile = blockIdx.x;
+  int cur = 0;
+  wait_vm0();
+  dma_tile(0, tile);  // the grid is at most tiles
+  wait_vm0();
+  __syncthreads();
+  for (; tile < tiles; tile += gridDim.x, cur ^= 1) {
+    if (tile + gridDim.x < tiles) dma_tile(cur ^ 1, tile + gridDim.x);
+    const char* sb = lds + cur * kLinTile + row * kC * 4;
+    int first = (hh ^ (row & 31)) << 4;
+    asm volatile("" : "+v"(first));  // the reads' 16 addresses again per tile: kept, they spill weights
+    f32x16 acc;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 b4 = *(const f32x4*)(sbias + c0 + 8 * q + 4 * hh);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[4 * q + e] = b4[e];
+    }
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const f32x4 x = *(const f32x4*)(sb + (first ^ (32 * j)));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[j][e], x[e], acc, 0, 0, 0);
+    }
+    const int64_t at = tile * kLinRows + row;
+    if (at < rows) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        store4(out + at * kC + c0 + 8 * q + 4 * hh, f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]});
+    }
+    wait_vm0();
+    __syncthreads();
+  }
+}
+
 struct Workspace {
   int64_t qg, kv, mterm, mflag, total;
 };
@@ -590,6 +656,18 @@ int bmx_triattn_fp32_fwd(const float* x, const float* mask, int64_t n, int start
   const int64_t items = (int64_t)kH * ((a.rows + kG - 1) / kG) * ((a.n + kCoreQ - 1) / kCoreQ);
   triattn_fp32_core_kernel<<<(unsigned)((items + 7) / 8 * 8), kCoreThreads, 0, stream>>>(c);
   return check_launch(fn);
+}
+
+int bmx_linear128_f32_fwd(const float* x, int64_t rows, const float* w, const float* b, float* out,
+                          hipStream_t stream) {
+  BMX_REQUIRE(rows >= 0, "bmx_linear128_f32_fwd: rows must be >= 0 (got %lld)", (long long)rows);
+  if (rows == 0) return BMX_OK;
+  BMX_REQUIRE(x && w && b && out, "bmx_linear128_f32_fwd: null pointer");
+  BMX_REQUIRE(((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)out) % 16 == 0,
+              "bmx_linear128_f32_fwd: pointers must be 16-byte aligned");
+  const int64_t tiles = (rows + kLinRows - 1) / kLinRows, most = 2 * device_cu_count();
+  linear128_f32_kernel<<<(unsigned)(tiles < most ? tiles : most), 64 * kLinWaves, 0, stream>>>(x, rows, w, b, out);
+  return check_launch("bmx_linear128_f32_fwd");
 }
 
 }  // extern "C"

@@ -109,6 +109,11 @@ def _f32(t):
     return t.detach().to(torch.float32).contiguous()
 
 
+def _aligned(t):
+    """``t``, copied where its storage offset leaves it short of 16-byte alignment."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def pack_mfma_weights(w):
     """bf16 copy of the row-major matrix ``w`` in MFMA A-operand order
     (``bmx_pack_mfma_weights``): each 32-row x 16-column operand tile becomes
@@ -683,8 +688,8 @@ def _triattn_fp32_native(module, x, mask, starting, tri_bias, stages, row0, rows
     """One ``bmx_triattn_fp32_fwd`` call on frame rows row0 .. row0 + rows - 1."""
     w, b, wb = _triattn_fp32_split_weights(module)
     ln = module.layer_norm
-    lnw = _f32(ln.weight)
-    lnb = None if ln.bias is None else _f32(ln.bias)
+    lnw = _aligned(_f32(ln.weight))
+    lnb = None if ln.bias is None else _aligned(_f32(ln.bias))
     N.call("bmx_triattn_fp32_fwd", x.data_ptr(), None if mask is None else mask.data_ptr(), x.shape[0], int(starting),
            row0, rows, float(module.inf), lnw.data_ptr(), None if lnb is None else lnb.data_ptr(), float(ln.eps),
            w.data_ptr(), b.data_ptr(), wb.data_ptr(), tri_bias.data_ptr(), stages,
@@ -711,7 +716,8 @@ def triattn_fp32(module, x, mask, starting, block_rows=None):
     (``bmx_triattn_fp32_fwd``; the ending node reads x's columns in place); the
     attention, mask bias, softmax, PV product and gate run fused on split-bf16
     products, two rows sharing each fetch of the [4, N, N] triangle bias, so the
-    [N, 4, N, N] scores never reach HBM; ``linear_o`` is an fp32 GEMM.  In exact fp32 mode the fp32
+    [N, 4, N, N] scores never reach HBM; ``linear_o`` runs in place on the fp32
+    matrix cores.  In exact fp32 mode the fp32
     LN128 kernel, fp32 GEMMs and the fp32-MFMA attention run instead.  Returns
     fp32 [N, N, 128].
 
@@ -752,26 +758,28 @@ def _triattn_fp32_split(module, x, mask, starting, rows):
     (all of them in one block: one kernel writes the triangle bias, which every
     row shares, beside the rows' operands; several blocks: a first pass writes
     it for all rows)."""
-    n, mha = x.shape[0], module.mha
+    n, x, lin = x.shape[0], _aligned(x), module.mha.linear_o
     m = None if mask is None else mask.to(torch.float32).contiguous()
     tri_bias = torch.empty(4, n, (n + 63) // 64 * 64, device=x.device, dtype=torch.float32)
     ws = _workspace(N.lib().bmx_triattn_fp32_workspace_bytes(n, rows), x.device)
-    w_o, b_o = mha.linear_o.weight.float(), mha.linear_o.bias.float()
+    w_o, b_o = _aligned(_f32(lin.weight)), _aligned(_f32(lin.bias))
+    out = torch.empty(n, n, C, device=x.device, dtype=torch.float32)  # the attention's output, then linear_o's
+
+    def linear_o(o):
+        N.call("bmx_linear128_f32_fwd", o.data_ptr(), o.shape[0] * n, w_o.data_ptr(), b_o.data_ptr(), o.data_ptr(),
+               _stream(x))
+
     if rows >= n:
-        o = torch.empty(n, n, C, device=x.device, dtype=torch.float32)
         if n:
-            _triattn_fp32_native(module, x, m, starting, tri_bias, 3, 0, n, o, ws)
-        del ws, tri_bias  # 2 KB per pair, before linear_o's output is allocated
-        out = torch.nn.functional.linear(o, w_o, b_o)
+            _triattn_fp32_native(module, x, m, starting, tri_bias, 3, 0, n, out, ws)
+            linear_o(out)
     else:
         rows -= rows % 2 if rows > 1 else 0  # the attention pairs rows: the pairs of one pass
         _triattn_fp32_native(module, x, m, starting, tri_bias, 1, 0, n)
-        o = torch.empty(rows, n, C, device=x.device, dtype=torch.float32)
-        out = torch.empty(n, n, C, device=x.device, dtype=torch.float32)  # the output frame
         for i0 in range(0, n, rows):
-            r = min(rows, n - i0)
-            _triattn_fp32_native(module, x, m, starting, tri_bias, 2, i0, r, o, ws)
-            torch.addmm(b_o, o[:r].view(-1, C), w_o.t(), out=out[i0:i0 + r].view(-1, C))
+            o = out[i0:i0 + rows]
+            _triattn_fp32_native(module, x, m, starting, tri_bias, 2, i0, o.shape[0], o, ws)
+            linear_o(o)
     return out if starting else out.transpose(0, 1)
 
 

@@ -165,6 +165,11 @@ int bmx_triattn_fp32_fwd(const float* x, const float* mask, int64_t n, int start
                          const float* b_qkvg, const void* w_bias, float* tri_bias, int stages, float* out,
                          void* workspace, size_t workspace_bytes, bmx_stream_t stream);
 
+/* out = x w^T + b for rows of 128 in fp32 (w [128, 128], b [128]): the linear_o of fp32-mode triangle
+ * attention (reference triangle.py:38-52).  out may be x. */
+int bmx_linear128_f32_fwd(const float* x, int64_t rows, const float* w, const float* b, float* out,
+                          bmx_stream_t stream);
+
 /* fp32 weight rows as a packed operand of the sequence stack's fp32 linears: per 32 rows and 8
  * columns one contiguous 1 KB run in MFMA order (lane (row % 32) + 32 (column % 8 / 4) holds 4
  * columns); 32-row tile t goes to packed tile tile0 + t * tile_stride.  rows a multiple of 32, k of

@@ -59,3 +59,21 @@ def test_fp32_attention_offsets(gpu, n, scale, closed):
     assert scale == 1.0 or top > 100
     # split products: 2^-16 relative each; an error of a score is a relative error of its probability
     assert err < max(1e-4, 2 * 2**-16 * top)
+
+
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 127, 40000])
+@pytest.mark.parametrize("in_place", [True, False])
+def test_linear128(gpu, rows, in_place):
+    from boltz_lumi_amd import _native as N
+
+    g = torch.Generator().manual_seed(rows)
+    x, w, b = (torch.randn(*s, generator=g).to(gpu) for s in ((rows + 1, 128), (128, 128), (128,)))
+    want = torch.nn.functional.linear(x.double(), w.double(), b.double())
+    out = x.clone() if in_place else torch.full_like(x, 7.0)
+    src = out if in_place else x
+    N.call("bmx_linear128_f32_fwd", src.data_ptr(), rows, w.data_ptr(), b.data_ptr(), out.data_ptr(),
+           torch.cuda.current_stream().cuda_stream)
+    # 128 fp32 products and sums: 128 * 2^-24 of the sum of magnitudes at most
+    bound = 128 * 2**-24 * (x.double().abs() @ w.double().abs().t() + b.double().abs())
+    assert ((out.double() - want).abs() <= bound)[:rows].all()
+    assert torch.equal(out[rows], x[rows] if in_place else torch.full_like(x[rows], 7.0))  # the row past the end
