@@ -265,7 +265,7 @@ constexpr int kKT = 64;  // keys per pipeline stage
 // instruction copies 1 KB, lane l to byte 16 l), so the K and V^T tiles are
 // dense and XOR-swizzled in 16-byte chunks instead of padded; the MFMA operand
 // reads of 16 consecutive lanes then hit 16 distinct 4-bank groups:
-//   K tile   (64 keys x 32 d)  key k, d chunk c (8 dims)  -> chunk 4k + (c ^ ((k >> 2) & 3))
+//   K tile   (64 keys x 32 d)  key k, d chunk c (8 dims)  -> chunk 4k + (c ^ chunk_swizzle(k))
 //   V^T tile (32 d x 64 keys)  dim d, key chunk c (8 keys) -> chunk 8d + (c ^ ((d >> 1) & 7))
 constexpr int kTileBytes = kKT * kD * 2;  // one K or V^T tile of one row
 
@@ -378,7 +378,7 @@ __device__ __forceinline__ bool core_rows(const Layout& L, int i0, int h, int q0
   for (int u = 0; u < 2; ++u) {
     const int job = w + 8 * u, r = job >> 3, kind = (job >> 2) & 1, quarter = job & 3;
     if (kind == 0) {
-      const int key = 16 * quarter + (l >> 2), c = (l & 3) ^ ((key >> 2) & 3);
+      const int key = 16 * quarter + (l >> 2), c = (l & 3) ^ chunk_swizzle(key);
       kv_src[u] = kb[r] + key * kD + 8 * c;
       kv_step[u] = kKT * kD;
     } else {
@@ -429,7 +429,7 @@ __device__ __forceinline__ bool core_rows(const Layout& L, int i0, int h, int q0
   if (g == (lq >> 3)) ident[lq & 7] = (bf16)1.f;
 
   // Per-lane LDS read offsets (bytes) inside a stage buffer.
-  const int k_rd = kOffK + (4 * lq + (g ^ ((lq >> 2) & 3))) * 16;  // + 1024 j (16 keys) + r tile
+  const int k_rd = kOffK + (4 * lq + (g ^ chunk_swizzle(lq))) * 16;  // + 1024 j (16 keys) + r tile
   const int b_rd = kOffBias + w * kBiasWaveBytes + 16 * (l & 31);   // + 512 j
 
   dma_stage(0, 0);

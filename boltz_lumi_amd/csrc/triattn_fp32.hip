@@ -30,11 +30,11 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
 
 // K and V^T of one (row, head): a record of four 2 KB tiles per 32-key block, K
 // high, K low ([key][dim]), V^T high, V^T low ([dim][key slot]), each 32 rows of
-// four 16-byte chunks, chunk c of row r at position c ^ (r / 4 % 4): one LDS DMA
+// four 16-byte chunks, chunk c of row r at position c ^ chunk_swizzle(r): one LDS DMA
 // copies 1 KB of it as it lies, and the attention's reads (lane l: row l % 16,
 // chunk l / 16) meet no bank twice.
 constexpr int kTile = 2048, kRecord = 4 * kTile;
-__device__ __forceinline__ int tile_at(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4); }
+__device__ __forceinline__ int tile_at(int row, int chunk) { return row * 64 + ((chunk ^ chunk_swizzle(row)) << 4); }
 
 // Key slot inside a 32-key block: the attention's P operand order (slot 8 gi + e holds key 4 gi + e, or
 // 16 + 4 gi + e - 4 from e = 4 on).
