@@ -78,9 +78,12 @@ constexpr size_t kFoldBytes = 2 * kFoldHalf * sizeof(bf16) + 16 * sizeof(float);
 
 constexpr int kZRow = kC + 8;  // fp32 LDS row of the updated tile: 4 rows apart = 32 banks apart
 
-// Row p of the tile's updated fp32 rows, over the xn and hid tiles (adjacent:
-// TP fp32 rows fill them exactly).
-__device__ __forceinline__ float* zrow(bf16* smem, int p) { return (float*)smem + p * kZRow; }
+// Row p of the tile's TP updated fp32 rows: the first half over xn, the second over hid (two
+// arrays: as halves of one, the compiler orders hid's stores with xn's reads, 0.5-1% of the kernel).
+template <int TP>
+__device__ __forceinline__ float* zrow(bf16* xn, bf16* hid, int p) {
+  return (float*)(p < TP / 2 ? xn : hid) + p % (TP / 2) * kZRow;
+}
 
 // The rows are never normalised in place.  Wave w takes the 16-row tiles w, w +
 // 4, ...; lane (row l%16, group g) reads channels 32q + 8g .. +7
@@ -123,13 +126,13 @@ __device__ __forceinline__ PairBiasFrags load_pair_bias_frags(const bf16* fold) 
 }
 
 template <int TP>
-__device__ __forceinline__ void pair_bias_epilogue(bf16* smem, const PairBiasFrags& f, const PairBiasArgs& pb,
-                                                   int64_t r0, int64_t rows) {
+__device__ __forceinline__ void pair_bias_epilogue(bf16* xn, bf16* hid, const PairBiasFrags& f,
+                                                   const PairBiasArgs& pb, int64_t r0, int64_t rows) {
   const int l = lane_id(), w = threadIdx.x >> 6, g = l >> 4, hc = l & 15;
 #pragma unroll
   for (int j = 0; j < (TP + 63) / 64; ++j) {
     if (TP < 64 && 16 * w >= TP) break;  // wave-uniform
-    const float* row = zrow(smem, 16 * (w + 4 * j) + hc) + 8 * g;
+    const float* row = zrow<TP>(xn, hid, 16 * (w + 4 * j) + hc) + 8 * g;
     f32x4 xv[8];
 #pragma unroll
     for (int q = 0; q < 4; ++q) xv[2 * q] = *(const f32x4*)(row + 32 * q), xv[2 * q + 1] = *(const f32x4*)(row + 32 * q + 4);
@@ -191,9 +194,9 @@ __global__ __launch_bounds__(256, 2) void pair_transition_kernel(const TIn* x, c
                                                               const bf16* __restrict__ w3, void* out, int out_mode,
                                                               int64_t rows, PairBiasArgs pb) {
   constexpr int NT = TP / 32;
-  __shared__ __attribute__((aligned(16))) bf16 smem[2 * TP * kLdsRow];
-  bf16 *xn = smem, *hid = smem + TP * kLdsRow;
-  static_assert(2 * kLdsRow * sizeof(bf16) == kZRow * sizeof(float), "TP fp32 rows must fill xn and hid");
+  __shared__ __attribute__((aligned(16))) bf16 xn[TP * kLdsRow];
+  __shared__ __attribute__((aligned(16))) bf16 hid[TP * kLdsRow];
+  static_assert(2 * kLdsRow * sizeof(bf16) == kZRow * sizeof(float), "TP / 2 fp32 rows must fill xn, as many hid");
   const int64_t r0 = (int64_t)blockIdx.x * TP;
   const int t = threadIdx.x, l = lane_id(), w = t >> 6;
   const int c0 = 32 * w;  // this wave's 32 hidden channels of each chunk / 32 output channels
@@ -268,9 +271,9 @@ __global__ __launch_bounds__(256, 2) void pair_transition_kernel(const TIn* x, c
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) zrow(smem, nt * 32 + drow(r, l))[c0 + (l & 31)] = y[nt][r];
+      for (int r = 0; r < 16; ++r) zrow<TP>(xn, hid, nt * 32 + drow(r, l))[c0 + (l & 31)] = y[nt][r];
     __syncthreads();
-    pair_bias_epilogue<TP>(smem, pbf, pb, r0, rows);
+    pair_bias_epilogue<TP>(xn, hid, pbf, pb, r0, rows);
   }
 }
 
