@@ -30,9 +30,9 @@ def _native_shape_ok(module, x) -> bool:
 
 
 # fp32 mode holds at most this many bytes per pair at its peak (``ops.triattn_fp32``:
-# q, g and the split K / V, the triangle bias, the attention output and the
-# linear_o result; in exact fp32 mode the [N^2, 512] projection beside them), all
-# N rows at once.  Measured at N = 1024: 2584 bytes per pair by default,
+# q, g and the split K / V, the triangle bias and the attention output, which
+# linear_o overwrites; in exact fp32 mode the [N^2, 512] projection beside them), all
+# N rows at once.  Measured at N = 1024: 2580 bytes per pair by default,
 # 3088-3604 with exact fp32 linears (tests/test_gpu_fp32_triattn.py); the bound
 # keeps a margin.
 FP32_BYTES_PER_PAIR = 4608
