@@ -412,7 +412,13 @@ def _stack_pack(layer, d, inner):
 
 
 def _params(*modules):
-    return [p for m in modules for p in (m._parameters.get("weight"), m._parameters.get("bias")) if p is not None]
+    """The weights and biases of ``modules``, or None where one of them is not a
+    parameter that its module stores: a computed weight
+    (``torch.nn.utils.parametrize``, a wrapper's property) is another tensor on
+    every access, so a pack keyed on stored parameters would not see it change."""
+    if not all("weight" in m._parameters and "bias" in m._parameters for m in modules):
+        return None
+    return [p for m in modules for p in (m._parameters["weight"], m._parameters["bias"]) if p is not None]
 
 
 def _adaln_parts(adaln, c):
@@ -452,12 +458,12 @@ def _stack_layer(layer, d):
         return None
     akids = att._modules
     proj_o = akids["proj_o"]
-    inner = up.out_features
-    if (not _untouched(proj_o) or inner % 32 or tuple(sw._parameters["weight"].shape) != (2 * inner, d)
-            or tuple(down._parameters["weight"].shape) != (d, inner)):
-        return None
     sources = _params(*first[:3], *second[:3], gate, gate_t, akids["proj_q"], akids["proj_k"], akids["proj_v"],
                       akids["proj_g"], proj_o, sw, up, down)
+    inner = up.out_features
+    if (sources is None or not _untouched(proj_o) or inner % 32 or tuple(sw.weight.shape) != (2 * inner, d)
+            or tuple(down.weight.shape) != (d, inner)):
+        return None
     return att, first[3], second[3], first[0].eps, inner, sources
 
 

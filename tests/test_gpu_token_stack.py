@@ -5,6 +5,7 @@ import copy
 
 import pytest
 import torch
+import torch.nn.utils.parametrize as parametrize
 from torch import nn
 
 from boltz_lumi_amd import _native, adapters, diffusion, ops
@@ -100,4 +101,28 @@ def test_token_stack_leaves_other_cases(gpu):
     finally:
         ops.exact_fp32_linears(before)
     assert rel < 1e-5
+    assert "bmx_token_stack_fwd" not in calls
+
+
+class _Doubled(nn.Module):
+    def forward(self, w):
+        return 2 * w
+
+
+@pytest.mark.parametrize("path", ["pair_bias_attn.proj_q", "transition.swish_gate.0", "transition.b_to_a"])
+def test_token_stack_computed_weights(gpu, path):
+    """A parametrized linear keeps the per-layer path, which follows its
+    parameter from call to call."""
+    ref, stack = _stack(gpu)
+    calls = []
+    wrapped, plain = stack.layers[1].get_submodule(path), ref.layers[1].get_submodule(path)
+    parametrize.register_parametrization(wrapped, "weight", _Doubled())
+    with torch.no_grad():
+        plain.weight.mul_(2)
+    for _ in range(2):
+        rel, mx = _run(stack, ref, gpu, 1, 1, 40, calls)
+        assert rel < 3e-5 and mx < 1e-4
+        with torch.no_grad():
+            plain.weight.mul_(-0.75)
+            wrapped.parametrizations.weight.original.mul_(-0.75)
     assert "bmx_token_stack_fwd" not in calls
