@@ -358,6 +358,9 @@ def layer_forward(self, a, s, bias=None, mask=None, to_keys=None, multiplicity=1
 # call on its own few-row linears (bmx_token_stack_fwd); above, per layer on the
 # library's split-bf16 GEMMs (linear_x3.hip holds both sides' times).
 TOKEN_STACK_MAX_ROWS = 1024
+# Widest rows and transition that the call takes (its row passes hold a row of
+# 1024 in one wave, as the per-layer path's do).
+TOKEN_STACK_MAX_WIDTH, TOKEN_STACK_MAX_INNER = 1024, 1 << 20
 
 
 def _stack_pack(layer, d, inner):
@@ -461,7 +464,8 @@ def _stack_layer(layer, d):
     sources = _params(*first[:3], *second[:3], gate, gate_t, akids["proj_q"], akids["proj_k"], akids["proj_v"],
                       akids["proj_g"], proj_o, sw, up, down)
     inner = up.out_features
-    if (sources is None or not _untouched(proj_o) or inner % 32 or tuple(sw.weight.shape) != (2 * inner, d)
+    if (sources is None or not _untouched(proj_o) or d > TOKEN_STACK_MAX_WIDTH or inner % 32
+            or inner > TOKEN_STACK_MAX_INNER or tuple(sw.weight.shape) != (2 * inner, d)
             or tuple(down.weight.shape) != (d, inner)):
         return None
     return att, first[3], second[3], first[0].eps, inner, sources

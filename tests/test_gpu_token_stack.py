@@ -17,8 +17,8 @@ pytestmark = pytest.mark.gpu
 DEPTH, HEADS, WIDTH = 3, 16, 768
 
 
-def _stack(dev, biased=False):
-    ref = R.DiffusionTransformer(DEPTH, HEADS, WIDTH, WIDTH)
+def _stack(dev, biased=False, heads=HEADS, width=WIDTH):
+    ref = R.DiffusionTransformer(DEPTH, heads, width, width)
     if biased:  # every bias the call can carry, an s_norm with a bias among them
         ref.layers[1].adaln.s_norm = nn.LayerNorm(WIDTH)
         for layer in ref.layers:
@@ -38,8 +38,9 @@ def _stack(dev, biased=False):
 def _run(stack, ref, dev, structures, samples, n, calls):
     g = torch.Generator().manual_seed(n)
     b = structures * samples
-    a, s = torch.randn(b, n, WIDTH, generator=g).to(dev), torch.randn(b, n, WIDTH, generator=g).to(dev)
-    bias = torch.randn(structures, n, n, DEPTH * HEADS, generator=g).to(dev)
+    att = ref.layers[0].pair_bias_attn
+    a, s = torch.randn(b, n, att.c_s, generator=g).to(dev), torch.randn(b, n, att.c_s, generator=g).to(dev)
+    bias = torch.randn(structures, n, n, DEPTH * att.num_heads, generator=g).to(dev)
     mask = torch.ones(b, n, device=dev)
     if n > 4:
         mask[0, -3:] = 0
@@ -126,3 +127,11 @@ def test_token_stack_computed_weights(gpu, path):
             plain.weight.mul_(-0.75)
             wrapped.parametrizations.weight.original.mul_(-0.75)
     assert "bmx_token_stack_fwd" not in calls
+
+
+def test_token_stack_wide_rows(gpu):
+    """32 heads of 48 (1536 channels) are wider than the call's rows."""
+    ref, stack = _stack(gpu, heads=32, width=1536)
+    calls = []
+    rel, mx = _run(stack, ref, gpu, 1, 1, 40, calls)
+    assert rel < 3e-5 and mx < 1e-4 and "bmx_token_stack_fwd" not in calls

@@ -49,3 +49,12 @@ def test_token_stack_takes_stored_weights_only():
         assert accepted(layer) is None, name
         setattr(owner, name, kept)
     assert accepted(layer) is not None
+
+
+@pytest.mark.parametrize("heads,width,taken", [(16, 768, True), (32, 32 * 32, True), (32, 32 * 48, False),
+                                               (22, 22 * 48, False)])
+def test_token_stack_width_limit(heads, width, taken):
+    """The call takes rows of at most 1024; wider layers, which AttentionPairBias
+    alone would allow (64 heads of 48), keep the per-layer path."""
+    layer = token_stack(heads, width).layers[0]
+    assert (accepted(layer, width) is not None) == taken
