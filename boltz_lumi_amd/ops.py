@@ -1035,7 +1035,7 @@ def f32_pack(rows, k, *parts):
     (tile0, tile stride, weight)."""
     out = torch.empty(rows * k, device=parts[0][2].device, dtype=torch.float32)
     for tile0, stride, w in parts:
-        w = _f32(w)
+        w = _aligned(_f32(w))
         N.call("bmx_f32_pack", w.data_ptr(), w.shape[0], w.shape[1], w.stride(0), tile0, stride, out.data_ptr(),
                _stream(w))
     return out
@@ -1054,6 +1054,9 @@ def sequence_stack(s, params, eps_attn, eps_trans, bias, mask, heads, hidden, in
     _check(bias.shape == (b, heads, n, n) and bias.dtype == torch.float32 and bias.is_contiguous(),
            "expected a contiguous fp32 [B, H, N, N] bias")
     _check(mask.shape == (b, n) and mask.dtype == torch.float32 and mask.stride(1) == 1, "expected an fp32 [B, N] mask")
+    # views at an odd storage offset (slices of one flat buffer) are copied: the call reads 16 bytes at a time
+    s = _aligned(s)
+    params = [None if p is None else _aligned(p) for p in params]
     out = torch.empty_like(s)
     ws = _workspace(N.lib().bmx_sequence_stack_workspace_bytes(b * n, d, hidden), s.device)
     N.call("bmx_sequence_stack_fwd", s.data_ptr(), b, n, heads, d // heads, hidden,

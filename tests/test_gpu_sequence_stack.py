@@ -78,3 +78,23 @@ def test_sequence_stack_keeps_other_cases(gpu):
     with torch.inference_mode():
         got = pairformer.sequence_stack(mine, s, z, mask, pair_bias=bias)
         assert torch.allclose(got.double(), _want(ref, s, bias, mask), atol=1e-4, rtol=1e-4)
+
+
+def test_sequence_stack_odd_offsets(gpu):
+    """Contiguous fp32 activations and parameters at a 4-byte storage offset
+    (views of one flat buffer): the same result as at an aligned one."""
+
+    def offset(t):
+        return torch.empty(t.numel() + 1, device=gpu)[1:].view(t.shape).copy_(t)
+
+    _, mine = _layer(gpu)
+    s, bias = torch.randn(1, 40, 384, device=gpu), torch.randn(1, 16, 40, 40, device=gpu)
+    z, mask = torch.zeros(1, 40, 40, 128, device=gpu), torch.ones(1, 40, device=gpu)
+    with torch.inference_mode():
+        want = pairformer.sequence_stack(mine, s, z, mask, pair_bias=bias)
+    with torch.no_grad():
+        for module in mine.modules():
+            for name, p in list(module.named_parameters(recurse=False)):
+                setattr(module, name, torch.nn.Parameter(offset(p), requires_grad=False))
+        got = pairformer.sequence_stack(mine, offset(s), z, mask, pair_bias=bias)
+    assert torch.equal(got, want)

@@ -8,7 +8,7 @@ import torch
 import torch.nn.utils.parametrize as parametrize
 from torch import nn
 
-from boltz_lumi_amd import adapters, diffusion
+from boltz_lumi_amd import _native, adapters, diffusion, layers, ops, pairformer
 from oracle import boltz_ref as R
 
 
@@ -58,3 +58,55 @@ def test_token_stack_width_limit(heads, width, taken):
     alone would allow (64 heads of 48), keep the per-layer path."""
     layer = token_stack(heads, width).layers[0]
     assert (accepted(layer, width) is not None) == taken
+
+
+class Calls:
+    """``ops`` on CPU tensors with every native call recorded instead of made."""
+
+    def __init__(self, monkeypatch):
+        if not _native.lib_path().exists():
+            pytest.skip("libbmx.so not built")
+        self.made = []
+        monkeypatch.setattr(_native, "call", lambda name, *args: self.made.append((name, args)))
+        monkeypatch.setattr(ops, "_cuda", lambda *_: None)
+        monkeypatch.setattr(ops, "_stream", lambda _: 0)
+
+    def __getitem__(self, name):
+        return [args for made, args in self.made if made == name]
+
+
+def offset(t):
+    """``t``'s values as a contiguous view at a 4-byte storage offset."""
+    flat = torch.empty(t.numel() + 4)
+    start = next(i for i in range(1, 5) if (flat.data_ptr() + 4 * i) % 16 == 4)
+    return flat[start:start + t.numel()].view(t.shape).copy_(t)
+
+
+def sequence_layer():
+    layer = layers.PairformerLayer().eval()
+    for p in layer.parameters():
+        p.requires_grad_(False)
+    return layer
+
+
+def sequence_call(layer, s):
+    b, n = s.shape[:2]
+    params, hidden = pairformer._native_sequence_params(layer, s.device)
+    return ops.sequence_stack(s, params, 1e-5, 1e-5, torch.zeros(b, 16, n, n), torch.ones(b, n), 16, hidden, 1e6)
+
+
+def test_sequence_stack_operands_are_aligned(monkeypatch):
+    """Contiguous parameters and activations at any storage offset: what the call
+    gets is 16-byte aligned."""
+    layer, s = sequence_layer(), offset(torch.randn(1, 5, 384))
+    with torch.no_grad():
+        for module in layer.modules():
+            for name, p in list(module.named_parameters(recurse=False)):
+                setattr(module, name, nn.Parameter(offset(p), requires_grad=False))
+    assert all(p.data_ptr() % 16 == 4 for p in layer.attention.parameters())
+    calls = Calls(monkeypatch)
+    with torch.inference_mode():
+        sequence_call(layer, s)
+    assert len(calls["bmx_f32_pack"]) == 8 and all(args[0] % 16 == 0 for args in calls["bmx_f32_pack"])
+    (args,) = calls["bmx_sequence_stack_fwd"]
+    assert args[0] % 16 == 0 and all((p or 0) % 16 == 0 for p in args[6])
