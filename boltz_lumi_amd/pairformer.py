@@ -41,6 +41,8 @@ from . import ops
 from ._guards import bf16_autocast, fp32_contiguous_on, gfx950_tensor, inference
 
 MAX_N = 8192  # the fused triangle attention's limit
+# what ``ops.sequence_stack`` takes: batch elements, rows in all, hidden channels
+SEQUENCE_MAX_BATCH, SEQUENCE_MAX_ROWS, SEQUENCE_MAX_HIDDEN = 65535, 1 << 20, 1 << 16
 
 
 def _plain(module) -> bool:
@@ -238,6 +240,11 @@ def _own(module):
     return None if not _plain(module) or "forward" in module.__dict__ else module._parameters
 
 
+def _native_sequence_rows(batch, n) -> bool:
+    """``ops.sequence_stack`` takes ``batch`` elements of ``n`` rows."""
+    return 0 < batch <= SEQUENCE_MAX_BATCH and 0 < batch * n <= SEQUENCE_MAX_ROWS
+
+
 def _native_sequence_params(layer, device):
     """The 9 parameters of ``ops.sequence_stack`` where the whole sequence
     stack (``sequence_ok`` holds) may run as that one call: plain LayerNorms,
@@ -257,13 +264,15 @@ def _native_sequence_params(layer, device):
         return None
     if any(o.get("bias") is not None for o in own[3:]) or own[0].get("bias") is None or own[1].get("bias") is None:
         return None
+    if not (pre.eps > 0 and norm.eps > 0):  # torch's LayerNorm takes 0, the call does not
+        return None
     hidden = own[7]["weight"].shape[0]
     shapes = [(384,), (384,)] + [(384, 384)] * 5 + [(hidden, 384), (hidden, 384), (384, hidden)]
     weights = [o["weight"] for o in own]
     rest = [weights[0], own[0]["bias"], weights[1], own[1]["bias"]]
     q_bias = own[2].get("bias")
     sources = weights[2:]
-    if hidden % 32 or any(w.shape != shape for w, shape in zip(weights, shapes)):
+    if hidden % 32 or hidden > SEQUENCE_MAX_HIDDEN or any(w.shape != shape for w, shape in zip(weights, shapes)):
         return None
     for p in sources + rest + ([] if q_bias is None else [q_bias]):
         if p.dtype != torch.float32 or not p.is_contiguous() or p.device != device:
@@ -290,7 +299,7 @@ def sequence_stack(layer, s, z, mask, pair_bias=None):
         s = s.float()
         seq_ok = sequence_ok(layer, s, z, mask)
         if (seq_ok and pair_bias is not None and s.is_cuda and not torch.is_grad_enabled()
-                and not layer.training and s.shape[0] > 0 and s.shape[1] > 0):
+                and not layer.training and _native_sequence_rows(s.shape[0], s.shape[1])):
             params = _native_sequence_params(layer, s.device)
             if params is not None:
                 m, att = mask.float(), layer.attention

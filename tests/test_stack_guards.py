@@ -110,3 +110,16 @@ def test_sequence_stack_operands_are_aligned(monkeypatch):
     assert len(calls["bmx_f32_pack"]) == 8 and all(args[0] % 16 == 0 for args in calls["bmx_f32_pack"])
     (args,) = calls["bmx_sequence_stack_fwd"]
     assert args[0] % 16 == 0 and all((p or 0) % 16 == 0 for p in args[6])
+
+
+def test_sequence_stack_limits():
+    """What the call refuses (an eps of 0, more rows or hidden channels than it
+    takes) keeps torch's path, which runs it."""
+    layer = sequence_layer()
+    for norm in (layer.pre_norm_s, layer.transition_s.norm):
+        kept, norm.eps = norm.eps, 0.0
+        assert pairformer._native_sequence_params(layer, torch.device("cpu")) is None
+        norm.eps = kept
+    assert pairformer._native_sequence_rows(1, 1) and pairformer._native_sequence_rows(1 << 15, 32)
+    for b, n in ((0, 5), (5, 0), (65536, 1), (1, (1 << 20) + 1), ((1 << 15) + 1, 32)):
+        assert not pairformer._native_sequence_rows(b, n), (b, n)
