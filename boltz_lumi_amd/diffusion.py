@@ -371,6 +371,8 @@ def _stack_pack(layer, d, inner):
     dev = att.proj_q.weight.device
 
     def pack(rows, k, *parts):  # parts: (tile0, tile stride, weight, column scale)
+        ops._check(sum(w.shape[0] for _, _, w, _ in parts) == rows and all(w.shape[1] == k for _, _, w, _ in parts),
+                   "a projection does not match the stack's width")
         out = torch.empty(rows * k * 2, device=dev, dtype=torch.bfloat16)
         for tile0, stride, w, scale in parts:
             ops.x3_pack(out, tile0, w, stride, scale)
@@ -379,8 +381,10 @@ def _stack_pack(layer, d, inner):
     def biases(pairs):  # concatenated biases of (linear, bias or None); None when there is none
         if all(b is None for _, b in pairs):
             return None
+        ops._check(all(b is None or (b.device == dev and b.numel() == lin.weight.shape[0]) for lin, b in pairs),
+                   "a bias does not match its projection")
         return torch.cat([b.detach().float() if b is not None
-                          else lin.weight.new_zeros(lin.out_features, dtype=torch.float32) for lin, b in pairs])
+                          else lin.weight.new_zeros(lin.weight.shape[0], dtype=torch.float32) for lin, b in pairs])
 
     def cond(lin, sn):  # s_scale / s_bias of an AdaLN: the s_norm weight is the column scale, its bias folds into b
         b = lin.bias
@@ -506,6 +510,8 @@ def _native_stack(layers, a, s, bias, mask, multiplicity):
         if sbias is not None and stride != sbias:
             return None
         sbias = stride
+        if sources[0].get_device() != a.get_device():
+            return None
         pack = ops.cached_value(layers[i], "token_stack", sources, lambda: _stack_pack(layers[i], d, inner))
         keep += [zb, pack]
         addresses += [0 if t is None else t.data_ptr() for t in pack]

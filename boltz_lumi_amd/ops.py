@@ -493,6 +493,10 @@ def x3_pack(out, tile0, w, tile_stride=1, col_scale=None):
     """Weight rows ``w`` [N, K] (times ``col_scale`` [K] per column) into the
     packed split operand ``out`` (``bmx_x3_pack``): 32-row tile t at tile
     ``tile0 + t * tile_stride``."""
+    _cuda(out, w, *(() if col_scale is None else (col_scale,)))
+    _check(w.dim() == 2 and w.shape[0] % 32 == 0 and (col_scale is None or col_scale.shape == w.shape[1:])
+           and (tile0 + (w.shape[0] // 32 - 1) * tile_stride + 1) * 64 * w.shape[1] <= out.numel(),
+           "the weight's 32-row tiles do not fit the packed operand")
     w = _f32(w)
     scale = None if col_scale is None else _f32(col_scale)
     N.call("bmx_x3_pack", w.data_ptr(), w.shape[0], w.shape[1], w.stride(0), None if scale is None else scale.data_ptr(),
@@ -1033,6 +1037,10 @@ def seq_attention_windowed(q, k, v, bias, mask, g, inf, *, windows, key_offset, 
 def f32_pack(rows, k, *parts):
     """Packed fp32 operand of ``rows`` x ``k`` (``bmx_f32_pack``) from ``parts`` of
     (tile0, tile stride, weight)."""
+    _cuda(*(w for _, _, w in parts))
+    for tile0, stride, w in parts:
+        _check(w.dim() == 2 and w.shape[1] == k and w.shape[0] % 32 == 0
+               and (tile0 + (w.shape[0] // 32 - 1) * stride + 1) * 32 <= rows, "a weight does not fit the packed operand")
     out = torch.empty(rows * k, device=parts[0][2].device, dtype=torch.float32)
     for tile0, stride, w in parts:
         w = _aligned(_f32(w))

@@ -274,7 +274,10 @@ def _native_sequence_params(layer, device):
     sources = weights[2:]
     if hidden % 32 or hidden > SEQUENCE_MAX_HIDDEN or any(w.shape != shape for w, shape in zip(weights, shapes)):
         return None
-    for p in sources + rest + ([] if q_bias is None else [q_bias]):
+    vectors = rest + ([] if q_bias is None else [q_bias])
+    if any(v.shape != (384,) for v in vectors):
+        return None
+    for p in sources + vectors:
         if p.dtype != torch.float32 or not p.is_contiguous() or p.device != device:
             return None
 

@@ -63,12 +63,13 @@ def test_token_stack_width_limit(heads, width, taken):
 class Calls:
     """``ops`` on CPU tensors with every native call recorded instead of made."""
 
-    def __init__(self, monkeypatch):
+    def __init__(self, monkeypatch, devices=False):
         if not _native.lib_path().exists():
             pytest.skip("libbmx.so not built")
         self.made = []
         monkeypatch.setattr(_native, "call", lambda name, *args: self.made.append((name, args)))
-        monkeypatch.setattr(ops, "_cuda", lambda *_: None)
+        if not devices:
+            monkeypatch.setattr(ops, "_cuda", lambda *_: None)
         monkeypatch.setattr(ops, "_stream", lambda _: 0)
 
     def __getitem__(self, name):
@@ -123,3 +124,50 @@ def test_sequence_stack_limits():
     assert pairformer._native_sequence_rows(1, 1) and pairformer._native_sequence_rows(1 << 15, 32)
     for b, n in ((0, 5), (5, 0), (65536, 1), (1, (1 << 20) + 1), ((1 << 15) + 1, 32)):
         assert not pairformer._native_sequence_rows(b, n), (b, n)
+
+
+def test_packs_refuse_host_weights(monkeypatch):
+    """The packs hand raw addresses to a kernel: host tensors are refused."""
+    calls = Calls(monkeypatch, devices=True)
+    with pytest.raises(RuntimeError, match="CUDA"):
+        ops.x3_pack(torch.empty(2 * 32 * 64, dtype=torch.bfloat16), 0, torch.zeros(32, 64))
+    with pytest.raises(RuntimeError, match="CUDA"):
+        ops.f32_pack(32, 64, (0, 1, torch.zeros(32, 64)))
+    assert not calls.made
+
+
+def test_packs_refuse_what_does_not_fit(monkeypatch):
+    """A weight whose 32-row tiles lie past the packed operand, or of another
+    width, is refused before the kernel writes; the last tile that fits is not."""
+    calls = Calls(monkeypatch)
+    out = torch.empty(2 * 96 * 64, dtype=torch.bfloat16)  # three tiles of 32 x 64
+    ops.x3_pack(out, 1, torch.zeros(64, 64))
+    ops.x3_pack(out, 0, torch.zeros(64, 64), tile_stride=2, col_scale=torch.ones(64))
+    ops.f32_pack(96, 64, (0, 2, torch.zeros(64, 64)), (1, 1, torch.zeros(32, 64)))
+    assert len(calls.made) == 4
+    for tile0, stride, rows, cols, scale in ((2, 1, 64, 64, None), (1, 2, 64, 64, None), (0, 1, 96, 96, None),
+                                             (0, 1, 33, 64, None), (0, 1, 32, 64, 32)):
+        with pytest.raises(RuntimeError):
+            ops.x3_pack(out, tile0, torch.zeros(rows, cols), stride, None if scale is None else torch.ones(scale))
+    for tile0, stride, rows, cols in ((2, 1, 64, 64), (1, 2, 64, 64), (0, 1, 32, 96), (0, 1, 33, 64)):
+        with pytest.raises(RuntimeError):
+            ops.f32_pack(96, 64, (tile0, stride, torch.zeros(rows, cols)))
+    assert len(calls.made) == 4
+
+
+@pytest.mark.parametrize("path", ["pair_bias_attn.proj_k", "transition.a_to_b", "output_projection_linear"])
+def test_token_stack_refuses_mismatched_projections(monkeypatch, path):
+    """A projection of another output width fills only a part of its pack: it
+    is refused, as the per-layer path's GEMM refuses it."""
+    layer = token_stack().layers[0]
+    Calls(monkeypatch)
+    *parents, name = path.split(".")
+    owner = layer.get_submodule(".".join(parents))
+    kept = getattr(owner, name)
+    narrow = nn.Linear(kept.in_features, kept.out_features - 32, bias=kept.bias is not None)
+    narrow.out_features = kept.out_features
+    setattr(owner, name, narrow)
+    if path == "output_projection_linear":
+        layer.output_projection[0] = narrow
+    with torch.inference_mode(), pytest.raises(RuntimeError, match="does not match"):
+        diffusion._stack_pack(layer, 768, 1536)
