@@ -673,6 +673,9 @@ def _triattn_fp32_split_weights(module):
     lins = (mha.linear_q, mha.linear_k, mha.linear_v, mha.linear_g)
 
     def build():
+        shapes = [(C, C)] * 4 + [(4, C)]
+        _check(all(lin.weight.shape == shape and (lin.bias is None or lin.bias.shape == shape[:1])
+                   for lin, shape in zip(lins + (module.linear,), shapes)), "expected 128 -> 128 and 128 -> 4 projections")
         w = torch.empty(2 * 4 * C * C, device=mha.linear_q.weight.device, dtype=torch.bfloat16)
         for i, lin in enumerate(lins):
             x3_pack(w, i * C // 32, lin.weight)
@@ -694,6 +697,8 @@ def _triattn_fp32_native(module, x, mask, starting, tri_bias, stages, row0, rows
     ln = module.layer_norm
     lnw = _aligned(_f32(ln.weight))
     lnb = None if ln.bias is None else _aligned(_f32(ln.bias))
+    _cuda(x, w, b, wb, lnw, tri_bias, *(t for t in (mask, lnb, out, ws) if t is not None))
+    _check(lnw.shape == (C,) and (lnb is None or lnb.shape == (C,)), "expected a LayerNorm of 128 channels")
     N.call("bmx_triattn_fp32_fwd", x.data_ptr(), None if mask is None else mask.data_ptr(), x.shape[0], int(starting),
            row0, rows, float(module.inf), lnw.data_ptr(), None if lnb is None else lnb.data_ptr(), float(ln.eps),
            w.data_ptr(), b.data_ptr(), wb.data_ptr(), tri_bias.data_ptr(), stages,
@@ -763,10 +768,16 @@ def _triattn_fp32_split(module, x, mask, starting, rows):
     row shares, beside the rows' operands; several blocks: a first pass writes
     it for all rows)."""
     n, x, lin = x.shape[0], _aligned(x), module.mha.linear_o
-    m = None if mask is None else mask.to(torch.float32).contiguous()
+    m = None
+    if mask is not None:
+        _check(mask.dim() == 2 and mask.shape[1 if starting else 0] == n and mask.shape[0 if starting else 1] in (1, n),
+               "expected a mask of [N, N], or one row (starting) or column (ending) of it")
+        m = mask.to(torch.float32).expand(n, n).contiguous()
     tri_bias = torch.empty(4, n, (n + 63) // 64 * 64, device=x.device, dtype=torch.float32)
     ws = _workspace(N.lib().bmx_triattn_fp32_workspace_bytes(n, rows), x.device)
     w_o, b_o = _aligned(_f32(lin.weight)), _aligned(_f32(lin.bias))
+    _cuda(x, w_o, b_o)
+    _check(w_o.shape == (C, C) and b_o.shape == (C,), "expected a 128 -> 128 linear_o with a bias")
     out = torch.empty(n, n, C, device=x.device, dtype=torch.float32)  # the attention's output, then linear_o's
 
     def linear_o(o):

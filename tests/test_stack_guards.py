@@ -171,3 +171,53 @@ def test_token_stack_refuses_mismatched_projections(monkeypatch, path):
         layer.output_projection[0] = narrow
     with torch.inference_mode(), pytest.raises(RuntimeError, match="does not match"):
         diffusion._stack_pack(layer, 768, 1536)
+
+
+def fp32_call(module, x, mask, starting, rows=None):
+    n = x.shape[0]
+    with torch.inference_mode():
+        return ops._triattn_fp32_split(module, x, mask, starting, n if rows is None else rows)
+
+
+def test_fp32_triangle_attention_refuses_host_tensors(monkeypatch):
+    calls = Calls(monkeypatch, devices=True)
+    layer = R.TriangleAttention(128, 32, 4).eval()
+    with pytest.raises(RuntimeError, match="CUDA"):
+        fp32_call(layer, torch.zeros(5, 5, 128), None, True)
+    assert not calls.made
+
+
+def test_fp32_triangle_attention_masks(monkeypatch):
+    """[N, N], or one row for all rows of the frame (x's columns for the ending
+    node); the kernel reads N x N values. Other shapes are refused."""
+    calls = Calls(monkeypatch)
+    seen = []
+    real = ops._triattn_fp32_native
+    monkeypatch.setattr(ops, "_triattn_fp32_native", lambda m, x, mask, *a, **k: seen.append(mask) or real(m, x, mask, *a, **k))
+    n, row = 5, torch.rand(5)
+    for starting in (True, False):
+        layer = (R.TriangleAttention if starting else R.TriangleAttentionEndingNode)(128, 32, 4).eval()
+        x = torch.zeros(n, n, 128)
+        for mask in (torch.rand(n, n), torch.rand(n, n) > 0.5, row[None] if starting else row[:, None]):
+            fp32_call(layer, x, mask, starting)
+            got = seen.pop()
+            assert got.dtype == torch.float32 and got.is_contiguous() and torch.equal(got, mask.float().expand(n, n))
+        made = len(calls.made)
+        for mask in (row, torch.rand(n, n + 1), torch.rand(n + 1, n), row[:, None] if starting else row[None],
+                     torch.rand(1, n, n)):
+            with pytest.raises(RuntimeError, match="mask"):
+                fp32_call(layer, x, mask, starting)
+        assert len(calls.made) == made
+
+
+def test_fp32_triangle_attention_refuses_other_widths(monkeypatch):
+    calls = Calls(monkeypatch)
+    x = torch.zeros(5, 5, 128)
+    for path, module in (("mha.linear_k", nn.Linear(128, 96, bias=False)), ("linear", nn.Linear(128, 3, bias=False)),
+                         ("mha.linear_o", nn.Linear(96, 128)), ("layer_norm", nn.LayerNorm(64))):
+        layer = R.TriangleAttention(128, 32, 4).eval()
+        *parents, name = path.split(".")
+        setattr(layer.get_submodule(".".join(parents)), name, module)
+        with pytest.raises(RuntimeError, match="expected"):
+            fp32_call(layer, x, None, True)
+    assert not [name for name, _ in calls.made if name != "bmx_x3_pack"]
