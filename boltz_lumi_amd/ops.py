@@ -79,15 +79,20 @@ def cached_value(module, name: str, sources, build):
     ``torch.inference_mode``) carry no version counter, so an in-place update of
     one cannot be seen: with such a source the value is rebuilt on every call
     and never cached."""
-    try:
-        key = [(id(p), p._version, p.data_ptr(), p.dtype) for p in sources]
-    except RuntimeError:  # no version counter
-        if not any(p.is_inference() for p in sources):
-            raise
+    cache = module.__dict__.setdefault("_bmx_weight_cache", {})
+    hit, key = cache.get(name), None
+    # Reading a missing version counter raises, which costs 30 us; asking every source costs 0.2 us each.
+    # So inference sources are asked for while nothing is cached, and a cached value's are read at once.
+    if hit is not None or not any(p.is_inference() for p in sources):
+        try:
+            key = [(id(p), p._version, p.data_ptr(), p.dtype) for p in sources]
+        except RuntimeError:
+            if not any(p.is_inference() for p in sources):
+                raise
+            cache.pop(name, None)  # an inference tensor has taken a source's place
+    if key is None:
         with torch.no_grad():
             return build()
-    cache = module.__dict__.setdefault("_bmx_weight_cache", {})
-    hit = cache.get(name)
     if hit is None or hit[0] != key:
         with torch.no_grad():
             value = build()
