@@ -622,8 +622,8 @@ int bmx_triattn_fp32_fwd(const float* x, const float* mask, int64_t n, int start
   if (n == 0 || rows == 0) return BMX_OK;
   BMX_REQUIRE(x && ln_w && w_qkvg && b_qkvg && w_bias && tri_bias, "bmx_triattn_fp32_fwd: null pointer");
   BMX_REQUIRE(((uintptr_t)x | (uintptr_t)ln_w | (uintptr_t)ln_b | (uintptr_t)w_qkvg | (uintptr_t)b_qkvg |
-               (uintptr_t)w_bias) % 16 == 0,
-              "bmx_triattn_fp32_fwd: x and parameters must be 16-byte aligned");
+               (uintptr_t)w_bias | (uintptr_t)tri_bias) % 16 == 0,
+              "bmx_triattn_fp32_fwd: x, tri_bias and parameters must be 16-byte aligned");
   const Workspace ws = make_workspace(n, rows);
   if (stages & 2) {
     BMX_REQUIRE(out && workspace, "bmx_triattn_fp32_fwd: null pointer");

@@ -158,7 +158,8 @@ int bmx_x3_pack(const float* w, int64_t rows, int64_t k, int64_t ldw, const floa
  * [512 + 4], the last 4 the triangle bias's; w_bias: the triangle-bias rows as bf16 [high, low][16][128] (rows past 4 zero).  stages:
  * 1 writes the rows' triangle bias into tri_bias [4, n, n rounded up to 64] (log2 units, zero past
  * n), 2 attends (tri_bias complete) into out
- * [rows, n, 128], 3 both (all rows).  workspace (stage 2): bmx_triattn_fp32_workspace_bytes. */
+ * [rows, n, 128], 3 both (all rows).  x, tri_bias, out and parameters 16-byte aligned; workspace
+ * (stage 2): bmx_triattn_fp32_workspace_bytes, 256-byte aligned. */
 size_t bmx_triattn_fp32_workspace_bytes(int64_t n, int64_t rows);
 int bmx_triattn_fp32_fwd(const float* x, const float* mask, int64_t n, int starting, int64_t row0, int64_t rows,
                          float inf, const float* ln_w, const float* ln_b, float eps, const void* w_qkvg,

@@ -181,3 +181,87 @@ def test_operator_set_entry_points_reject_bad_arguments(lib):
 def test_call_raises_with_message(lib):
     with pytest.raises(N.BmxError, match="eps must be positive"):
         N.call("bmx_layernorm", None, None, None, 0.0, None, 0, 1, 4, None)
+
+
+def test_one_call_entry_points_reject_bad_arguments(lib):
+    # The packs, the fp32-mode triangle attention, its output linear and the one-call stacks: alignment, sizes,
+    # short workspaces and missing parameters are refused before a launch; empty inputs are not.
+    fake, odd, eps = ctypes.c_void_p(256), ctypes.c_void_p(260), ctypes.c_float(1e-5)
+
+    def refused(rc, text):
+        return rc == N.BMX_EINVAL and text in lib.bmx_last_error()
+
+    assert lib.bmx_x3_pack(None, 0, 64, 64, None, 0, 1, None, None) == N.BMX_OK
+    assert refused(lib.bmx_x3_pack(fake, 33, 64, 64, None, 0, 1, fake, None), b"multiple of 32")
+    assert refused(lib.bmx_x3_pack(fake, 32, 64, 63, None, 0, 1, fake, None), b"ldw >= k")
+    assert refused(lib.bmx_x3_pack(fake, 32, 64, 64, None, 0, 0, fake, None), b"tile_stride >= 1")
+    assert refused(lib.bmx_x3_pack(fake, 32, 64, 64, None, 0, 1, odd, None), b"16-byte aligned")
+    assert lib.bmx_f32_pack(None, 0, 64, 64, 0, 1, None, None) == N.BMX_OK
+    assert refused(lib.bmx_f32_pack(fake, 32, 60, 64, 0, 1, fake, None), b"multiple of 8")
+    for w, out in ((odd, fake), (fake, odd)):
+        assert refused(lib.bmx_f32_pack(w, 32, 64, 64, 0, 1, out, None), b"16-byte aligned")
+
+    assert lib.bmx_linear128_f32_fwd(None, 0, None, None, None, None) == N.BMX_OK
+    for i in range(4):
+        p = [odd if i == j else fake for j in range(4)]
+        assert refused(lib.bmx_linear128_f32_fwd(p[0], 5, p[1], p[2], p[3], None), b"16-byte aligned")
+
+    # x, mask, n, starting, row0, rows, inf, ln_w, ln_b, eps, w_qkvg, b_qkvg, w_bias, tri_bias, stages, out, ws, bytes
+    n = 100
+    need = lib.bmx_triattn_fp32_workspace_bytes(n, n)
+    good = [fake, None, n, 1, 0, n, 1e9, fake, None, eps, fake, fake, fake, fake, 3, fake, fake, need, None]
+
+    def triattn(**changed):
+        args = list(good)
+        for i, v in changed.items():
+            args[int(i[1:])] = v
+        return lib.bmx_triattn_fp32_fwd(*args)
+
+    assert triattn(_2=0, _5=0) == N.BMX_OK and triattn(_5=0, _14=2) == N.BMX_OK
+    for i in ("_0", "_7", "_8", "_10", "_11", "_12", "_13"):
+        assert refused(triattn(**{i: odd}), b"x, tri_bias and parameters must be 16-byte aligned"), i
+    assert refused(triattn(_15=odd), b"out must be 16-byte aligned")
+    assert refused(triattn(_16=ctypes.c_void_p(272)), b"256-byte")
+    assert refused(triattn(_17=need - 1), b"hold")
+    assert refused(triattn(_4=1), b"inside [0, n)")
+    assert refused(triattn(_5=50), b"for all rows, 3")
+    assert refused(triattn(_2=32769, _5=32769), b"[0, 32768]")
+    assert refused(triattn(_9=ctypes.c_float(0)), b"eps")
+    assert refused(triattn(_13=None), b"null pointer")
+
+    # s, batch, n, heads, head_dim, hidden, params, eps, eps, bias, mask, smask, inf, out, workspace, bytes
+    need = lib.bmx_sequence_stack_workspace_bytes(2 * 40, 384, 1536)
+
+    def sequence(params=None, s=fake, batch=2, n=40, heads=16, dim=24, hidden=1536, e=eps, out=fake, ws=fake, size=need):
+        params = (ctypes.c_void_p * 9)(*(params or [256] * 9))
+        return lib.bmx_sequence_stack_fwd(s, batch, n, heads, dim, hidden, params, e, eps, fake, fake, n, 1e6, out, ws,
+                                          size, None)
+
+    assert sequence(batch=0) == N.BMX_OK and sequence(n=0) == N.BMX_OK
+    for i in range(9):
+        assert refused(sequence([260 if j == i else 256 for j in range(9)]), b"16-byte aligned")
+        if i != 3:  # proj_q's bias may be absent
+            assert refused(sequence([None if j == i else 256 for j in range(9)]), b"null parameter")
+    assert refused(sequence(s=odd), b"16-byte aligned") and refused(sequence(out=odd), b"16-byte aligned")
+    assert refused(sequence(size=need - 1), b"too small") and refused(sequence(dim=40), b"head_dim")
+    assert refused(sequence(heads=24), b"at most 512") and refused(sequence(hidden=1500), b"multiples of 32")
+    assert refused(sequence(n=(1 << 19) + 1), b"2^20") and refused(sequence(e=ctypes.c_float(0)), b"eps")
+
+    # a, s, batch, n, heads, head_dim, inner, layers, params, eps_s, eps, mask, smask, sbias, bias_div, inf, out, ...
+    need = lib.bmx_token_stack_workspace_bytes(2, 300, 16, 48, 1536)
+
+    def token(params=None, a=fake, batch=2, n=300, heads=16, dim=48, inner=1536, layers=2, ws=fake, size=need):
+        params = (ctypes.c_void_p * 22)(*(params or [256] * 22))
+        return lib.bmx_token_stack_fwd(a, fake, batch, n, heads, dim, inner, layers, params, eps, (ctypes.c_float * 4)(
+            *[1e-5] * 4), fake, 0, 0, 1, 1e6, fake, ws, size, None)
+
+    assert token(batch=0) == N.BMX_OK and token(layers=0) == N.BMX_OK
+    for i in range(22):
+        if i % 11 != 10:  # the pair bias is read at any alignment
+            assert refused(token([260 if j == i else 256 for j in range(22)]), b"16-byte aligned")
+        if i % 11 == 10 or i % 2 == i // 11 % 2:  # weights and pair biases; the five biases may be absent
+            assert refused(token([None if j == i else 256 for j in range(22)]), b"null parameter")
+    assert refused(token(a=odd), b"16-byte aligned") and refused(token(ws=ctypes.c_void_p(272)), b"256-byte")
+    assert refused(token(size=need - 1), b"hold") and refused(token(n=513), b"[0, 1024]")
+    assert refused(token(heads=32), b"at most 1024") and refused(token(inner=1500), b"multiple of 32")
+    assert refused(token(dim=40), b"head_dim") and refused(token(heads=65, dim=24), b"heads must be")
