@@ -156,7 +156,7 @@ __global__ __launch_bounds__(64 * W) void linear_f32_kernel(LinearF32 a) {
     if constexpr (SWIGLU) {
       const f32x4 g = sum(r, 32 + c);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = v[i] / (1.f + __expf(-v[i])) * g[i];
+      for (int i = 0; i < 4; ++i) v[i] = v[i] / (1.f + expf(-v[i])) * g[i];  // __expf: an error of |v| ulp
     }
     if (a.bias && n < a.n_bias) v += load4(a.bias + n);
     if (a.res) v += load4(a.res + (int64_t)m * a.ldo + n);

@@ -98,3 +98,30 @@ def test_sequence_stack_odd_offsets(gpu):
                 setattr(module, name, torch.nn.Parameter(offset(p), requires_grad=False))
         got = pairformer.sequence_stack(mine, offset(s), z, mask, pair_bias=bias)
     assert torch.equal(got, want)
+
+
+def test_sequence_stack_silu(gpu):
+    """silu(v) * g alone in the output (one nonzero weight per row, no residual)
+    for v down to -80: as exact as fp32 operations give it. A fast exponential's
+    argument error grows with |v|."""
+    _, mine = _layer(gpu)
+    tr, v = mine.transition_s, -torch.arange(8, 8 + 384, device=gpu) * 0.2
+    scale = torch.exp2(torch.round(-v * 1.4427))  # a power of two: the product's rounding alone
+    with torch.no_grad():
+        for p in (mine.attention.proj_o.weight, tr.norm.weight, tr.fc1.weight, tr.fc2.weight, tr.fc3.weight):
+            p.zero_()
+        tr.norm.bias.fill_(1)
+        tr.fc1.weight[:384, 0] = v
+        tr.fc2.weight[:384, 0] = scale
+        tr.fc3.weight[:, :384] = torch.eye(384, device=gpu)
+    calls, real = [], _native.call
+    with torch.inference_mode(), pytest.MonkeyPatch.context() as mp:
+        mp.setattr(_native, "call", lambda name, *args: calls.append(name) or real(name, *args))
+        got = pairformer.sequence_stack(mine, torch.zeros(1, 40, 384, device=gpu),
+                                        torch.zeros(1, 40, 40, 128, device=gpu), torch.ones(1, 40, device=gpu),
+                                        pair_bias=torch.zeros(1, 16, 40, 40, device=gpu))
+    assert "bmx_sequence_stack_fwd" in calls
+    want = torch.nn.functional.silu(v.double()) * scale.double()
+    err = ((got.double() - want) / want).abs().max().item()
+    print(f"silu error {err:.2e}", flush=True)
+    assert err < 6 * 2**-24  # exp: 1 ulp; sum, quotient and product: half an ulp each
