@@ -41,8 +41,13 @@ from . import ops
 from ._guards import bf16_autocast, fp32_contiguous_on, gfx950_tensor, inference
 
 MAX_N = 8192  # the fused triangle attention's limit
-# what ``ops.sequence_stack`` takes: batch elements, rows in all, hidden channels
-SEQUENCE_MAX_BATCH, SEQUENCE_MAX_ROWS, SEQUENCE_MAX_HIDDEN = 65535, 1 << 20, 1 << 16
+# Up to this many rows (batch x tokens) the sequence stack runs as one native
+# call on its own fp32 linears; above, on the library's fp32 GEMMs (ten
+# launches), whose larger tiles then win: 1134 tokens 177 us against 194, 1536
+# 230 against 227, 2048 357 against 323, 4 x 512 212 against 193, 64 x 64 337
+# against 267.
+SEQUENCE_MAX_ROWS = 1280
+SEQUENCE_MAX_HIDDEN = 1 << 16  # hidden channels that the call takes
 
 
 def _plain(module) -> bool:
@@ -241,8 +246,8 @@ def _own(module):
 
 
 def _native_sequence_rows(batch, n) -> bool:
-    """``ops.sequence_stack`` takes ``batch`` elements of ``n`` rows."""
-    return 0 < batch <= SEQUENCE_MAX_BATCH and 0 < batch * n <= SEQUENCE_MAX_ROWS
+    """``batch`` elements of ``n`` rows run as one ``ops.sequence_stack`` call."""
+    return 0 < batch * n <= SEQUENCE_MAX_ROWS
 
 
 def _native_sequence_params(layer, device):

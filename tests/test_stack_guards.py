@@ -114,16 +114,16 @@ def test_sequence_stack_operands_are_aligned(monkeypatch):
 
 
 def test_sequence_stack_limits():
-    """What the call refuses (an eps of 0, more rows or hidden channels than it
-    takes) keeps torch's path, which runs it."""
+    """What the call refuses (an eps of 0) and rows past its line keep torch's path."""
     layer = sequence_layer()
     for norm in (layer.pre_norm_s, layer.transition_s.norm):
         kept, norm.eps = norm.eps, 0.0
         assert pairformer._native_sequence_params(layer, torch.device("cpu")) is None
         norm.eps = kept
-    assert pairformer._native_sequence_rows(1, 1) and pairformer._native_sequence_rows(1 << 15, 32)
-    for b, n in ((0, 5), (5, 0), (65536, 1), (1, (1 << 20) + 1), ((1 << 15) + 1, 32)):
-        assert not pairformer._native_sequence_rows(b, n), (b, n)
+    line = pairformer.SEQUENCE_MAX_ROWS
+    for b, n, native in ((1, 1, True), (1, line, True), (line // 64, 64, True), (line, 1, True), (0, 5, False), (5, 0, False),
+                         (1, line + 1, False), (line // 64 + 1, 64, False), (65536, 32, False)):
+        assert pairformer._native_sequence_rows(b, n) == native, (b, n)
 
 
 def test_packs_refuse_host_weights(monkeypatch):
