@@ -696,17 +696,16 @@ def _triattn_fp32_split_weights(module):
     return cached_value(module, "fp32_proj_x3", srcs, build)
 
 
-def _triattn_fp32_native(module, x, mask, starting, tri_bias, stages, row0, rows, out=None, ws=None):
-    """One ``bmx_triattn_fp32_fwd`` call on frame rows row0 .. row0 + rows - 1."""
-    w, b, wb = _triattn_fp32_split_weights(module)
-    ln = module.layer_norm
-    lnw = _aligned(_f32(ln.weight))
-    lnb = None if ln.bias is None else _aligned(_f32(ln.bias))
+def _triattn_fp32_native(module, weights, x, mask, starting, tri_bias, stages, row0, rows, out=None, ws=None):
+    """One ``bmx_triattn_fp32_fwd`` call on frame rows row0 .. row0 + rows - 1;
+    ``weights``: ``_triattn_fp32_split_weights`` and the LayerNorm's weight and
+    bias (or None)."""
+    w, b, wb, lnw, lnb = weights
     _cuda(x, w, b, wb, lnw, tri_bias, *(t for t in (mask, lnb, out, ws) if t is not None))
     _check(lnw.shape == (C,) and (lnb is None or lnb.shape == (C,)), "expected a LayerNorm of 128 channels")
     N.call("bmx_triattn_fp32_fwd", x.data_ptr(), None if mask is None else mask.data_ptr(), x.shape[0], int(starting),
-           row0, rows, float(module.inf), lnw.data_ptr(), None if lnb is None else lnb.data_ptr(), float(ln.eps),
-           w.data_ptr(), b.data_ptr(), wb.data_ptr(), tri_bias.data_ptr(), stages,
+           row0, rows, float(module.inf), lnw.data_ptr(), None if lnb is None else lnb.data_ptr(),
+           float(module.layer_norm.eps), w.data_ptr(), b.data_ptr(), wb.data_ptr(), tri_bias.data_ptr(), stages,
            None if out is None else out.data_ptr(), None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
            _stream(x))
 
@@ -781,6 +780,9 @@ def _triattn_fp32_split(module, x, mask, starting, rows):
     tri_bias = torch.empty(4, n, (n + 63) // 64 * 64, device=x.device, dtype=torch.float32)
     ws = _workspace(N.lib().bmx_triattn_fp32_workspace_bytes(n, rows), x.device)
     w_o, b_o = _aligned(_f32(lin.weight)), _aligned(_f32(lin.bias))
+    ln = module.layer_norm
+    weights = (*_triattn_fp32_split_weights(module), _aligned(_f32(ln.weight)),
+               None if ln.bias is None else _aligned(_f32(ln.bias)))
     _cuda(x, w_o, b_o)
     _check(w_o.shape == (C, C) and b_o.shape == (C,), "expected a 128 -> 128 linear_o with a bias")
     out = torch.empty(n, n, C, device=x.device, dtype=torch.float32)  # the attention's output, then linear_o's
@@ -791,14 +793,14 @@ def _triattn_fp32_split(module, x, mask, starting, rows):
 
     if rows >= n:
         if n:
-            _triattn_fp32_native(module, x, m, starting, tri_bias, 3, 0, n, out, ws)
+            _triattn_fp32_native(module, weights, x, m, starting, tri_bias, 3, 0, n, out, ws)
             linear_o(out)
     else:
         rows -= rows % 2 if rows > 1 else 0  # the attention pairs rows: the pairs of one pass
-        _triattn_fp32_native(module, x, m, starting, tri_bias, 1, 0, n)
+        _triattn_fp32_native(module, weights, x, m, starting, tri_bias, 1, 0, n)
         for i0 in range(0, n, rows):
             o = out[i0:i0 + rows]
-            _triattn_fp32_native(module, x, m, starting, tri_bias, 2, i0, o.shape[0], o, ws)
+            _triattn_fp32_native(module, weights, x, m, starting, tri_bias, 2, i0, o.shape[0], o, ws)
             linear_o(o)
     return out if starting else out.transpose(0, 1)
 

@@ -193,7 +193,7 @@ def test_fp32_triangle_attention_masks(monkeypatch):
     calls = Calls(monkeypatch)
     seen = []
     real = ops._triattn_fp32_native
-    monkeypatch.setattr(ops, "_triattn_fp32_native", lambda m, x, mask, *a, **k: seen.append(mask) or real(m, x, mask, *a, **k))
+    monkeypatch.setattr(ops, "_triattn_fp32_native", lambda m, w, x, mask, *a: seen.append(mask) or real(m, w, x, mask, *a))
     n, row = 5, torch.rand(5)
     for starting in (True, False):
         layer = (R.TriangleAttention if starting else R.TriangleAttentionEndingNode)(128, 32, 4).eval()
@@ -221,3 +221,17 @@ def test_fp32_triangle_attention_refuses_other_widths(monkeypatch):
         with pytest.raises(RuntimeError, match="expected"):
             fp32_call(layer, x, None, True)
     assert not [name for name, _ in calls.made if name != "bmx_x3_pack"]
+
+
+@pytest.mark.parametrize("n,rows", [(9, 9), (9, 4), (9, 1)])
+def test_fp32_triangle_attention_packs_once_per_call(monkeypatch, n, rows):
+    """Inference-tensor weights carry no version counter, so every call packs
+    them again: once, however many blocks of rows it runs in."""
+    calls = Calls(monkeypatch)
+    with torch.inference_mode():
+        layer = R.TriangleAttention(128, 32, 4).eval()
+        for _ in range(2):
+            calls.made.clear()
+            ops._triattn_fp32_split(layer, torch.zeros(n, n, 128), None, True, rows)
+            assert len(calls["bmx_x3_pack"]) == 4
+            assert len(calls["bmx_linear128_f32_fwd"]) == -(-n // rows)
