@@ -484,6 +484,9 @@ def _native_stack(layers, a, s, bias, mask, multiplicity):
     b, n, d = a.shape
     if d % 32 or a.shape != s.shape or not ops.use_split(d) or not 0 < b * n <= TOKEN_STACK_MAX_ROWS or mask is None:
         return None
+    # a bias that prepare_token_bias has not packed: before the walk over the layers, 20 us each
+    if bias.dtype != torch.float32 or (n > 1 and bias.stride()[1:3] != (n, 1)):
+        return None
     parts = []
     for layer in layers:
         part = _stack_layer(layer, d)

@@ -35,7 +35,7 @@ def _stack(dev, biased=False, heads=HEADS, width=WIDTH):
     return ref, host.structure_module.score_model.token_transformer
 
 
-def _run(stack, ref, dev, structures, samples, n, calls):
+def _run(stack, ref, dev, structures, samples, n, calls, pack=prepare_token_bias):
     g = torch.Generator().manual_seed(n)
     b = structures * samples
     att = ref.layers[0].pair_bias_attn
@@ -48,8 +48,8 @@ def _run(stack, ref, dev, structures, samples, n, calls):
     real = _native.call
     with torch.inference_mode(), pytest.MonkeyPatch.context() as mp:
         mp.setattr(_native, "call", lambda name, *args: calls.append(name) or real(name, *args))
-        got = stack(a, s, prepare_token_bias(bias), mask, None, samples)
-        again = stack(a, s, prepare_token_bias(bias), mask, None, samples)
+        got = stack(a, s, pack(bias), mask, None, samples)
+        again = stack(a, s, pack(bias), mask, None, samples)
         want = ref(a, s, bias, mask, None, samples)
     assert torch.equal(a, a0) and torch.equal(got, again)
     return ((got - want).double().norm() / want.double().norm()).item(), (got - want).abs().max() / want.abs().max()
@@ -102,6 +102,9 @@ def test_token_stack_leaves_other_cases(gpu):
     finally:
         ops.exact_fp32_linears(before)
     assert rel < 1e-5
+    for n in (1, 2, 40):  # upstream's layout; at one token it is the packed one
+        rel, mx = _run(stack, ref, gpu, 1, 1, n, calls if n > 1 else [], pack=lambda bias: bias)
+        assert rel < 3e-5 and mx < 1e-4
     assert "bmx_token_stack_fwd" not in calls
 
 

@@ -9,6 +9,7 @@ import torch.nn.utils.parametrize as parametrize
 from torch import nn
 
 from boltz_lumi_amd import _native, adapters, diffusion, layers, ops, pairformer
+from boltz_lumi_amd.pair_bias import prepare_token_bias
 from oracle import boltz_ref as R
 
 
@@ -235,3 +236,31 @@ def test_fp32_triangle_attention_packs_once_per_call(monkeypatch, n, rows):
             ops._triattn_fp32_split(layer, torch.zeros(n, n, 128), None, True, rows)
             assert len(calls["bmx_x3_pack"]) == 4
             assert len(calls["bmx_linear128_f32_fwd"]) == -(-n // rows)
+
+
+def test_token_stack_bias_layout(monkeypatch):
+    """Only a bias as ``prepare_token_bias`` packs it goes to the call, which
+    reads it as dense [heads, N, N] elements; another one is seen before the
+    layers are looked at."""
+    stack, n = token_stack(depth=2), 6
+    Calls(monkeypatch)
+    walked, given = [], []
+    real = diffusion._stack_layer
+    monkeypatch.setattr(diffusion, "_stack_layer", lambda *a: walked.append(1) or real(*a))
+    monkeypatch.setattr(diffusion, "_stack_pack", lambda *_: (None,) * 10)
+    monkeypatch.setattr(ops, "token_stack", lambda a, s, addresses, *_: given.append(addresses[10::11]) or a)
+    a, mask = torch.zeros(2, n, 768), torch.ones(2, n)
+    raw = torch.randn(1, n, n, 32)
+
+    def call(bias):
+        walked.clear()
+        given.clear()
+        with torch.inference_mode():
+            diffusion._native_stack(list(stack.layers), a, a, bias.view(1, n, n, 2, 16), mask, 2)
+        return bool(given), len(walked)
+
+    packed = prepare_token_bias(raw)
+    assert call(packed) == (True, 2)
+    assert given[0] == [packed.data_ptr(), packed.data_ptr() + 4 * 16 * n * n]
+    for other in (raw, raw.transpose(1, 2).contiguous().transpose(1, 2), packed.transpose(1, 2), packed.double()):
+        assert call(other) == (False, 0)
