@@ -3,13 +3,16 @@
 // split-bf16 attention.  Upstream's fp32 forward is TriangleAttention with
 // autocast off (reference triangle.py:38-52).
 //
-// What bounds the projection: HBM.  The projection reads 512 B and writes 2.1 KB per pair
-// (q and g fp32, K and V^T as bf16 high / low parts).  As separate passes (LayerNorm
+// What bounds the projection: HBM, and next the matrix cores.  The projection reads 512 B and writes 2.1 KB
+// per pair (q and g fp32, K and V^T as bf16 high / low parts).  As separate passes (LayerNorm
 // to a split operand, library GEMM to fp32 rows, a bias permute, the K / V split)
-// the same step moved 7 KB per pair: 751 us at n = 576, this kernel 178 (4.8
-// TB/s).
-// Products are split bf16 (xh wh + xl wh + xh wl, about 2^-16 relative), as the
-// library GEMM's were.
+// the same step moved 7 KB per pair: 751 us at n = 576, this kernel 199 (4.3
+// TB/s; 174 with three products).
+// Products are split bf16, all four of them in the projections (xl wl + xh wh + xl wh + xh wl), three in the
+// attention (about 2^-16 relative).  The fourth pays for the attention's offsets: whole numbers, so the largest
+// probability of a row is no longer exactly 1 and has a split error too.  Against 64 bits, mean of n = 17 .. 576:
+// 7.3e-6 with the separate passes, 7.7e-6 with three products here, 6.6e-6 with four (at every size below the
+// separate passes; four for v and g alone are not).
 #include "bmx_common.h"
 
 using namespace bmx;
@@ -57,7 +60,7 @@ struct ProjArgs {
 // Persistent and weight-stationary: 16 waves keep 32 output rows each (8 k steps,
 // high and low: 64 VGPRs), one block per CU, the next tile's rows prefetched into
 // registers.  (8 waves of 64 rows spilled at 256 VGPRs, and a scratch reload
-// waits for every prefetch and store before it: 347 us against 178.)  q, k, g come as D[output][pair] (4 consecutive
+// waits for every prefetch and store before it: twice the time.)  q, k, g come as D[output][pair] (4 consecutive
 // channels per lane), v as D[pair][dim] (4 consecutive keys).  q and g leave as
 // 16-byte stores, K and V^T through an LDS stage stored in the next iteration
 // before the next prefetch (vmcnt counts stores in issue order).
@@ -170,6 +173,7 @@ __global__ __launch_bounds__(64 * kWaves) void triattn_fp32_proj_kernel(ProjArgs
 #pragma unroll
           for (int ks = 0; ks < 8; ++ks) {
             const bf16x8 fh = frag(xh, kLdsRow, nt * 32, ks), fl = frag(xl, kLdsRow, nt * 32, ks);
+            acc = mfma32(fl, wl[ks], acc);
             acc = mfma32(fh, wh[ks], acc);
             acc = mfma32(fl, wh[ks], acc);
             acc = mfma32(fh, wl[ks], acc);
@@ -194,6 +198,7 @@ __global__ __launch_bounds__(64 * kWaves) void triattn_fp32_proj_kernel(ProjArgs
 #pragma unroll
           for (int ks = 0; ks < 8; ++ks) {
             const bf16x8 fh = frag(xh, kLdsRow, nt * 32, ks), fl = frag(xl, kLdsRow, nt * 32, ks);
+            acc = mfma32(wl[ks], fl, acc);
             acc = mfma32(wh[ks], fh, acc);
             acc = mfma32(wh[ks], fl, acc);
             acc = mfma32(wl[ks], fh, acc);
@@ -233,6 +238,7 @@ __global__ __launch_bounds__(64 * kWaves) void triattn_fp32_proj_kernel(ProjArgs
         const int ox = (16 * w + lq) * kLdsRow + 32 * ks + 8 * g, ow = lq * kLdsRow + 32 * ks + 8 * g;
         const bf16x8 fh = *(const bf16x8*)(xh + ox), fl = *(const bf16x8*)(xl + ox);
         const bf16x8 bh = *(const bf16x8*)(wb + ow), bl = *(const bf16x8*)(wb + 16 * kLdsRow + ow);
+        ab = mfma16(bl, fl, ab);
         ab = mfma16(bh, fh, ab);
         ab = mfma16(bh, fl, ab);
         ab = mfma16(bl, fh, ab);
