@@ -346,7 +346,8 @@ int sequence_attention_packed(const float* proj, int64_t batch, int64_t n, int h
 // lanes 0-31 first 0-3, 12-15, 20-27, then the others; lane l reads row l % 16, chunk l / 16, so
 // the row quads 0, 3 of one chunk and 1, 2 of its neighbour meet and must hold four different positions:
 // 0, 2, 3, 1 for the quads in turn (r / 4 % 4 itself gives two pairs of equal ones: 45% of the fp32 attention's
-// LDS cycles were conflicts, now none; 500 -> 480 us at n = 576, the bf16 core 936 -> 922 at n = 1024).
+// LDS cycles were conflicts, now none; 500 -> 480 us at n = 576; the bf16 core 936 -> 922 at n = 1024, which a
+// whole call's spread covers).
 __host__ __device__ inline int chunk_swizzle(int row) {
   const int q = row >> 2;
   return ((q ^ (q >> 1)) & 1) << 1 | ((q >> 1) & 1);

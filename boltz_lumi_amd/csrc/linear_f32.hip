@@ -13,8 +13,11 @@
 // the texture pipe, not the matrix cores, sets the time (fc1 | fc2 at 1134 rows 69
 // us against 54, at 117 17.5 against 13.5).  The rows a LayerNorm stands in
 // front of are normalised by each block into LDS in that order; activations
-// and residuals are the epilogue.  The stack's kernels, before (torch) and after:
-// 117 tokens 64 -> 48 us, 312 tokens 85 -> 68, 1134 tokens 223 -> 210.
+// and residuals are the epilogue.  The whole stack, before (torch, bound by the
+// host up to some 1200 rows) and after: 117 tokens 199 -> 49 us, 312 198 -> 64,
+// 1024 197 -> 141, 1280 195 -> 181; its kernels alone 64 -> 48 us at 117 tokens,
+// 223 -> 210 at 1134.  From about 1536 rows on the library's larger tiles win
+// (pairformer.py draws the line).
 #include "bmx_common.h"
 
 using namespace bmx;
@@ -175,12 +178,17 @@ int launch_linear(const char* name, LinearF32 a, hipStream_t stream) {
   const bool wide = SWIGLU || tiles > 700;
   a.tiles_n = !SWIGLU && wide ? (nt + 1) / 2 : nt;
   const dim3 grid((unsigned)(8 * (((int64_t)a.tiles_m * a.tiles_n + 7) / 8)));
-  if (SWIGLU || wide)
+  if (SWIGLU || wide) {
     linear_f32_kernel<2, 4, LN, SWIGLU><<<grid, 256, 0, stream>>>(a);
-  else if (a.k >= 1024)
-    linear_f32_kernel<1, 8, LN, false><<<grid, 512, 0, stream>>>(a);
-  else
-    linear_f32_kernel<1, 4, LN, false><<<grid, 256, 0, stream>>>(a);
+    return check_launch(name);
+  }
+  if constexpr (!LN) {  // normalised rows are at most kMaxLn wide
+    if (a.k >= 1024) {
+      linear_f32_kernel<1, 8, LN, false><<<grid, 512, 0, stream>>>(a);
+      return check_launch(name);
+    }
+  }
+  linear_f32_kernel<1, 4, LN, false><<<grid, 256, 0, stream>>>(a);
   return check_launch(name);
 }
 

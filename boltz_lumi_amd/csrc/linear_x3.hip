@@ -17,7 +17,10 @@
 // split-bf16 GEMM in brackets): 117 x 768 x 768 4.1 us (21), 117 x 3072 x 768
 // 5.3 (21), 117 x 768 x 1536 5.8 (24), 512 x 3072 x 768 11.8 (21), 1024 x 768 x
 // 768 7.5 (21), 1024 x 3072 x 768 21 (22), 2048 x 3072 x 768 48 (34): the line
-// to the library GEMM lies at 1024 rows (kMaxRows).
+// to the library GEMM lies at 1024 rows (kMaxRows).  Whole stacks of 24 layers on
+// either side of it, one call here and per-layer calls in brackets (bound by the
+// host, 11 launches a layer): 117 rows 1.6 ms (7.2), 512 3.1 (6.9), 1024 5.1
+// (6.5 .. 7.0), 5 x 204 4.5 (7.2); 1025 rows by per-layer calls 6.5.
 #include "bmx_common.h"
 
 using namespace bmx;
@@ -144,11 +147,11 @@ __global__ __launch_bounds__(64 * kW) void linear_x3_kernel(LinearArgs a) {
 int launch_linear(const char* name, LinearArgs a, hipStream_t stream) {
   a.tiles_m = (a.m + 31) / 32;
   const int nt = a.n / 32;
-  // 32-wide tiles while that is at most three blocks a CU, 64-wide ones (one
+  // 32-wide tiles while that is at most three blocks per CU, 64-wide ones (one
   // read of the x tile for two weight tiles) above: 117 x 768: 4.1 us against
   // 4.9, 1024 x 768: 7.5 against 8.5, 512 x 3072: 12.7 against 11.8, 1024 x 3072:
   // 24 against 21.
-  const bool wide = (int64_t)a.tiles_m * nt > 768;
+  const bool wide = (int64_t)a.tiles_m * nt > 3 * device_cu_count();
   a.tiles_n = a.op ? nt / 3 : wide ? (nt + 1) / 2 : nt;
   if (!a.x2) a.x2 = a.x, a.tile_split = nt;
   const dim3 grid(8 * ((a.tiles_m * a.tiles_n + 7) / 8)), block(64 * kW);

@@ -33,7 +33,10 @@ namespace {
 // the contraction the padded area: at n = 312 (512 instead of 320) 56 and 37 us
 // against 31 and 20, at n = 1134 360 and 533 us against 308 and 449.
 constexpr int kPlaneTile = 64;
-constexpr int kWorkspaceTile = 256;  // padding the workspace query counts (more than the planes use)
+// Padding that the workspace query counts: more than the planes use, kept from the 256-padded planes, so that
+// callers with sizes of their own still match it.  The modules share one workspace with triangle attention, whose
+// planes are padded to 256 and larger.
+constexpr int kWorkspaceTile = 256;
 
 // ------------------------------------------------------------------ K1
 // Persistent and weight-stationary: each wave keeps its [p_in; g_in] rows for
@@ -566,12 +569,14 @@ int launch(const float* x, const float* mask, int ni, int outgoing, const float*
   if (stages & 2) {
     // Tile by plane size.  256 x 256 tiles re-read the operands least and are
     // the fastest where they fill the chip (128 channels x 4 tiles from np = 512
-    // on) and either fit exactly (np = 512: 42 us against 47 in 128-wide tiles,
-    // 1024: 289 against 347) or their cut edge tiles are few (896: 232 against
-    // 245, 1152: 449 against 493).  In between 128-wide tiles win (np = 320: 20
-    // us against 26, 448: 38 and 38, 576: 70 against 84), and 64-wide ones at
-    // np <= 128, where they are the only ones with a block for every CU (117
-    // tokens: 4.7 us against 5.6).
+    // on) and either fit exactly (np = 512: 44 us against 45 in 128-wide tiles,
+    // 768: 142 against 161, 1024: 288 against 342) or their cut edge tiles are
+    // few (704: 127 against 135, 896: 228 against 237, 960: 272 against 301,
+    // 1152: 451 against 477).  Below, 128-wide tiles win (np = 320: 21 us against
+    // 26, 384: 26 against 31, 576: 74 against 87, 640: 99 against 104; only 448
+    // has 43 against 38, no slower than the 512-padded planes before), and
+    // 64-wide ones at np <= 128, where they are the only ones with a block for
+    // every CU (117 tokens: 4.7 us against 5.6).
     if (np > 640 || np == 512)
       launch_contract<256, 64, 128>(a_pl, b_pl, o_pl, np, 1, stream);
     else if (np > 128)

@@ -297,7 +297,8 @@ def layernorm_split3(x, eps):
 def layernorm_split3_t(x, eps):
     """``layernorm_split3`` of the rows of ``x.transpose(0, 1)`` for a square
     pair frame x [N, N, k] with dense rows, without the transposed copy
-    (``bmx_layernorm_split3_t_bf16``); bf16 [N, N, 3 k + 64]."""
+    (``bmx_layernorm_split3_t_bf16``); bf16 [N, N, 3 k + 64].  Part of the
+    public operator set; no module of this package calls it any more."""
     _cuda(x)
     _check(x.dim() == 3 and x.shape[0] == x.shape[1] and x.dtype == torch.float32 and x.is_contiguous()
            and 0 < x.shape[-1] <= 1024 and x.shape[-1] % 4 == 0,
@@ -760,7 +761,7 @@ def triattn_fp32(module, x, mask, starting, block_rows=None):
     tri_bias = tri_bias.permute(2, 0, 1).contiguous()  # [H, q, k], shared by every row
     m = x.new_ones(n, n) if mask is None else mask.to(torch.float32).contiguous()
     q, k, v, g = proj.split(C, dim=-1)
-    o = seq_attention_batched(q, k, v, tri_bias[None], m, g, module.inf, bias_div=n, split=not _EXACT_FP32[0])
+    o = seq_attention_batched(q, k, v, tri_bias[None], m, g, module.inf, bias_div=n, split=False)
     del q, k, v, g, proj, tri_bias  # 2.3 KB per pair, before linear_o's output is allocated
     out = torch.nn.functional.linear(o, mha.linear_o.weight.float(), mha.linear_o.bias.float())
     return out if starting else out.transpose(0, 1)
@@ -841,8 +842,7 @@ def _triattn_fp32_blocked(module, x, mask, starting, rows):
     for i0, i1 in blocks:
         proj = torch.nn.functional.linear(features(i0, i1), w, b).view(i1 - i0, n, -1)
         q, k, v, g = proj.split(C, dim=-1)
-        o = seq_attention_batched(q, k, v, tri_bias[None], m[i0:i1], g, module.inf, bias_div=i1 - i0,
-                                  split=not _EXACT_FP32[0])
+        o = seq_attention_batched(q, k, v, tri_bias[None], m[i0:i1], g, module.inf, bias_div=i1 - i0, split=False)
         del q, k, v, g, proj
         torch.addmm(b_o, o.view(-1, C), w_o.t(), out=out[i0:i1].view(-1, C))
         del o
