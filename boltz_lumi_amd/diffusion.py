@@ -371,7 +371,7 @@ def _stack_pack(layer, d, inner):
     dev = att.proj_q.weight.device
 
     def pack(rows, k, *parts):  # parts: (tile0, tile stride, weight, column scale)
-        ops._check(sum(w.shape[0] for _, _, w, _ in parts) == rows and all(w.shape[1] == k for _, _, w, _ in parts),
+        ops._check(sum(w.shape[0] * (w.shape[1] == k) for _, _, w, _ in parts) == rows,
                    "a projection does not match the stack's width")
         out = torch.empty(rows * k * 2, device=dev, dtype=torch.bfloat16)
         for tile0, stride, w, scale in parts:
@@ -381,10 +381,11 @@ def _stack_pack(layer, d, inner):
     def biases(pairs):  # concatenated biases of (linear, bias or None); None when there is none
         if all(b is None for _, b in pairs):
             return None
-        ops._check(all(b is None or (b.device == dev and b.numel() == lin.weight.shape[0]) for lin, b in pairs),
+        out = torch.cat([b.detach().float() if b is not None
+                         else lin.weight.new_zeros(lin.out_features, dtype=torch.float32) for lin, b in pairs])
+        ops._check(out.device == dev and out.numel() == sum(lin.weight.shape[0] for lin, _ in pairs),
                    "a bias does not match its projection")
-        return torch.cat([b.detach().float() if b is not None
-                          else lin.weight.new_zeros(lin.weight.shape[0], dtype=torch.float32) for lin, b in pairs])
+        return out
 
     def cond(lin, sn):  # s_scale / s_bias of an AdaLN: the s_norm weight is the column scale, its bias folds into b
         b = lin.bias

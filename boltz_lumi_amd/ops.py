@@ -499,14 +499,18 @@ def x3_pack(out, tile0, w, tile_stride=1, col_scale=None):
     """Weight rows ``w`` [N, K] (times ``col_scale`` [K] per column) into the
     packed split operand ``out`` (``bmx_x3_pack``): 32-row tile t at tile
     ``tile0 + t * tile_stride``."""
-    _cuda(out, w, *(() if col_scale is None else (col_scale,)))
-    _check(w.dim() == 2 and w.shape[0] % 32 == 0 and (col_scale is None or col_scale.shape == w.shape[1:])
-           and (tile0 + (w.shape[0] // 32 - 1) * tile_stride + 1) * 64 * w.shape[1] <= out.numel(),
+    w, rows, k = _f32(w), *w.shape
+    scale = None
+    if col_scale is not None:
+        scale = _f32(col_scale)
+        _check(scale.shape == (k,), "expected one column scale per column")
+        _cuda(out, scale)
+    if out.get_device() != w.get_device() or not w.is_cuda:
+        _cuda(out, w)
+    _check(rows % 32 == 0 and (tile0 + (rows // 32 - 1) * tile_stride + 1) * 64 * k <= out.numel(),
            "the weight's 32-row tiles do not fit the packed operand")
-    w = _f32(w)
-    scale = None if col_scale is None else _f32(col_scale)
-    N.call("bmx_x3_pack", w.data_ptr(), w.shape[0], w.shape[1], w.stride(0), None if scale is None else scale.data_ptr(),
-           tile0, tile_stride, out.data_ptr(), _stream(w))
+    N.call("bmx_x3_pack", w.data_ptr(), rows, k, k, None if scale is None else scale.data_ptr(), tile0, tile_stride,
+           out.data_ptr(), _stream(w))
 
 
 MODULATION, GATE, GATED_SWIGLU = 0, 1, 3
