@@ -679,38 +679,39 @@ def triattn(module, x, mask, starting, out_mode=OUT_BF16, out=None, workspace=No
 
 
 def _triattn_fp32_split_weights(module):
-    """fp32 mode's projections for ``bmx_triattn_fp32_fwd``: q | k | v | g packed
-    as a split operand, their biases and the triangle bias's [512 + 4], and the
-    triangle-bias rows as bf16 [high, low][16][128]."""
-    mha = module.mha
-    lins = (mha.linear_q, mha.linear_k, mha.linear_v, mha.linear_g)
+    """fp32 mode's weights: q | k | v | g packed as a split operand, their biases
+    and the triangle bias's [512 + 4], the triangle-bias rows as bf16 [high,
+    low][16][128], the LayerNorm's weight and bias (or None) and linear_o's."""
+    mha, ln, lo = module.mha, module.layer_norm, module.mha.linear_o
+    lins = (mha.linear_q, mha.linear_k, mha.linear_v, mha.linear_g, module.linear)
 
     def build():
-        shapes = [(C, C)] * 4 + [(4, C)]
+        shapes = [(C, C)] * 4 + [(4, C), (C, C)]
         _check(all(lin.weight.shape == shape and (lin.bias is None or lin.bias.shape == shape[:1])
-                   for lin, shape in zip(lins + (module.linear,), shapes)), "expected 128 -> 128 and 128 -> 4 projections")
-        w = torch.empty(2 * 4 * C * C, device=mha.linear_q.weight.device, dtype=torch.bfloat16)
-        for i, lin in enumerate(lins):
+                   for lin, shape in zip(lins + (lo,), shapes)) and lo.bias is not None,
+               "expected 128 -> 128 and 128 -> 4 projections and a linear_o with a bias")
+        _check(ln.weight.shape == (C,) and (ln.bias is None or ln.bias.shape == (C,)),
+               "expected a LayerNorm of 128 channels")
+        _cuda(*srcs)
+        w = torch.empty(2 * 4 * C * C, device=lo.weight.device, dtype=torch.bfloat16)
+        for i, lin in enumerate(lins[:4]):
             x3_pack(w, i * C // 32, lin.weight)
         b = torch.cat([lin.bias.detach().float() if lin.bias is not None
-                       else lin.weight.new_zeros(lin.out_features, dtype=torch.float32)
-                       for lin in lins + (module.linear,)])
+                       else lin.weight.new_zeros(lin.out_features, dtype=torch.float32) for lin in lins])
         rows = module.linear.weight.detach().float()
         rows = torch.cat([rows, rows.new_zeros(16 - rows.shape[0], C)])
         hi = rows.to(torch.bfloat16)
-        return w, b, torch.stack([hi, (rows - hi.float()).to(torch.bfloat16)]).contiguous()
+        return (w, b, torch.stack([hi, (rows - hi.float()).to(torch.bfloat16)]).contiguous(),
+                *(None if t is None else _aligned(_f32(t)) for t in (ln.weight, ln.bias, lo.weight, lo.bias)))
 
-    srcs = tuple(t for lin in lins + (module.linear,) for t in (lin.weight, lin.bias) if t is not None)
+    srcs = [t for lin in lins + (ln, lo) for t in (lin.weight, lin.bias) if t is not None]
     return cached_value(module, "fp32_proj_x3", srcs, build)
 
 
 def _triattn_fp32_native(module, weights, x, mask, starting, tri_bias, stages, row0, rows, out=None, ws=None):
     """One ``bmx_triattn_fp32_fwd`` call on frame rows row0 .. row0 + rows - 1;
-    ``weights``: ``_triattn_fp32_split_weights`` and the LayerNorm's weight and
-    bias (or None)."""
-    w, b, wb, lnw, lnb = weights
-    _cuda(x, w, b, wb, lnw, tri_bias, *(t for t in (mask, lnb, out, ws) if t is not None))
-    _check(lnw.shape == (C,) and (lnb is None or lnb.shape == (C,)), "expected a LayerNorm of 128 channels")
+    ``weights``: ``_triattn_fp32_split_weights``."""
+    w, b, wb, lnw, lnb = weights[:5]
     N.call("bmx_triattn_fp32_fwd", x.data_ptr(), None if mask is None else mask.data_ptr(), x.shape[0], int(starting),
            row0, rows, float(module.inf), lnw.data_ptr(), None if lnb is None else lnb.data_ptr(),
            float(module.layer_norm.eps), w.data_ptr(), b.data_ptr(), wb.data_ptr(), tri_bias.data_ptr(), stages,
@@ -779,20 +780,20 @@ def _triattn_fp32_split(module, x, mask, starting, rows):
     (all of them in one block: one kernel writes the triangle bias, which every
     row shares, beside the rows' operands; several blocks: a first pass writes
     it for all rows)."""
-    n, x, lin = x.shape[0], _aligned(x), module.mha.linear_o
-    m = None
+    n, x, m = x.shape[0], _aligned(x), None
     if mask is not None:
-        _check(mask.dim() == 2 and mask.shape[1 if starting else 0] == n and mask.shape[0 if starting else 1] in (1, n),
-               "expected a mask of [N, N], or one row (starting) or column (ending) of it")
-        m = mask.to(torch.float32).expand(n, n).contiguous()
+        if mask.shape != x.shape[:2]:
+            _check(mask.shape == ((1, n) if starting else (n, 1)),
+                   "expected a mask of [N, N], or one row (starting) or column (ending) of it")
+            mask = mask.expand(n, n)
+        m = mask.to(torch.float32).contiguous()
     tri_bias = torch.empty(4, n, (n + 63) // 64 * 64, device=x.device, dtype=torch.float32)
     ws = _workspace(N.lib().bmx_triattn_fp32_workspace_bytes(n, rows), x.device)
-    w_o, b_o = _aligned(_f32(lin.weight)), _aligned(_f32(lin.bias))
-    ln = module.layer_norm
-    weights = (*_triattn_fp32_split_weights(module), _aligned(_f32(ln.weight)),
-               None if ln.bias is None else _aligned(_f32(ln.bias)))
-    _cuda(x, w_o, b_o)
-    _check(w_o.shape == (C, C) and b_o.shape == (C,), "expected a 128 -> 128 linear_o with a bias")
+    weights = _triattn_fp32_split_weights(module)
+    w_o, b_o = weights[5:]
+    for t in (w_o,) if m is None else (w_o, m):  # all weights are on one device
+        if t.get_device() != x.get_device():
+            _cuda(x, t)
     out = torch.empty(n, n, C, device=x.device, dtype=torch.float32)  # the attention's output, then linear_o's
 
     def linear_o(o):
