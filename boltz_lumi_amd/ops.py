@@ -1088,13 +1088,15 @@ def sequence_stack(s, params, eps_attn, eps_trans, bias, mask, heads, hidden, in
     _check(bias.shape == (b, heads, n, n) and bias.dtype == torch.float32 and bias.is_contiguous(),
            "expected a contiguous fp32 [B, H, N, N] bias")
     _check(mask.shape == (b, n) and mask.dtype == torch.float32 and mask.stride(1) == 1, "expected an fp32 [B, N] mask")
-    # views at an odd storage offset (slices of one flat buffer) are copied: the call reads 16 bytes at a time
-    s = _aligned(s)
-    params = [None if p is None else _aligned(p) for p in params]
+    s, addresses = _aligned(s), [0 if p is None else p.data_ptr() for p in params]
+    if any(address % 16 for address in addresses):
+        # views at an odd storage offset (slices of one flat buffer): the call reads 16 bytes at a time
+        params = [None if p is None else _aligned(p) for p in params]
+        addresses = [0 if p is None else p.data_ptr() for p in params]
     out = torch.empty_like(s)
     ws = _workspace(N.lib().bmx_sequence_stack_workspace_bytes(b * n, d, hidden), s.device)
     N.call("bmx_sequence_stack_fwd", s.data_ptr(), b, n, heads, d // heads, hidden,
-           (ctypes.c_void_p * 9)(*[0 if p is None else p.data_ptr() for p in params]), float(eps_attn),
+           (ctypes.c_void_p * 9)(*addresses), float(eps_attn),
            float(eps_trans), bias.data_ptr(), mask.data_ptr(), mask.stride(0) if b > 1 else 0, float(inf),
            out.data_ptr(), ws.data_ptr(), ws.numel(), _stream(s))
     return out

@@ -280,10 +280,11 @@ def _native_sequence_params(layer, device):
     if hidden % 32 or hidden > SEQUENCE_MAX_HIDDEN or any(w.shape != shape for w, shape in zip(weights, shapes)):
         return None
     vectors = rest + ([] if q_bias is None else [q_bias])
-    if any(v.shape != (384,) for v in vectors):
+    if any(v.numel() != 384 for v in vectors):
         return None
+    index = -1 if device.type == "cpu" else device.index
     for p in sources + vectors:
-        if p.dtype != torch.float32 or not p.is_contiguous() or p.device != device:
+        if p.dtype != torch.float32 or not p.is_contiguous() or p.get_device() != index:
             return None
 
     def build():
