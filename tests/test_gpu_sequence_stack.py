@@ -57,8 +57,9 @@ def test_sequence_stack_rows(gpu, b, n):
     native = b * n <= pairformer.SEQUENCE_MAX_ROWS
     assert calls.count("bmx_sequence_stack_fwd") == (2 if native else 0)
     assert torch.equal(got, again) and torch.equal(s, s0)
-    err = lambda x: ((x.double() - want).norm() / want.norm()).item()
-    assert err(got) < max(1.5 * err(torch_path), 1e-6), (err(got), err(torch_path))
+    err, err_torch = (((x.double() - want).norm() / want.norm()).item() for x in (got, torch_path))
+    print(f"b={b} n={n}: {err:.2e}, torch {err_torch:.2e}", flush=True)
+    assert err <= max(err_torch, 2**-23)  # an ulp of the outputs: what one rounding more may cost
 
 
 def test_sequence_stack_keeps_other_cases(gpu):
